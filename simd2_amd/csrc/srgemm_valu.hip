@@ -7,7 +7,8 @@
 //     BN/(TN/4) columns apart so that every LDS read is one ds_read_b128 and
 //     the 16 (or more) lanes reading one row of Y hit distinct banks;
 //   * K advances in BK-deep slabs, double-buffered in LDS: the next slab's
-//     global loads (128-bit, coalesced along K for X and along columns for Y)
+//     global loads (16 bytes a lane at any row alignment, coalesced along K
+//     for X and along columns for Y)
 //     are issued before the current slab's arithmetic and written to the
 //     other LDS buffer afterwards, one barrier per slab;
 //   * X is stored transposed in LDS (k-major, padded by 4 floats so the
@@ -20,6 +21,7 @@
 // Tiles are walked XCD-aware: the 8 XCDs receive workgroups round-robin, so
 // each XCD is handed one contiguous range of tiles, and inside it tiles are
 // visited in groups of GROUP tile-rows so neighbours share panels in L2.
+#include <cmath>
 #include <mutex>
 
 #include "valu_tile.hpp"
@@ -28,15 +30,13 @@ namespace simd2 {
 
 namespace {
 
-// Launch forms: FAST -- the problem is a whole number of tiles and slabs and
-// every operand is 16-byte aligned row by row; SPLIT -- aligned, but the
-// shape is off the grid: tiles inside the matrix run the 128-bit path (their
-// last, partial K slab checked), the edge tiles the guarded 128-bit path
-// (rows past R read as padding, a column group past Cn element by element,
-// stores masked); CHECKED -- per-element bounds everywhere.
-enum { FORM_FAST = 0, FORM_SPLIT = 1, FORM_CHECKED = 2 };
-
-template <class Op, int BM, int BN, int TM, int TN, int BK, int WAVES, int FORM>
+// OFFGRID: the shape is not a whole number of tiles and slabs.  Tiles inside
+// the matrix differ only in the last, partial K slab, which is loaded element
+// by element with the op's padding; edge tiles keep 16-byte loads wherever a
+// 4-float group lies inside the matrix (rows past R read as padding, a column
+// group past Cn element by element) and mask their stores.  Rows need no
+// alignment (valu_tile.hpp).
+template <class Op, int BM, int BN, int TM, int TN, int BK, int WAVES, bool OFFGRID>
 __global__ __launch_bounds__((BM / TM) * (BN / TN))
 __attribute__((amdgpu_waves_per_eu(WAVES))) void srgemm_valu_kernel(
     int R, int Cn, int K, const float *__restrict__ X, int64_t ldx,
@@ -48,15 +48,12 @@ __attribute__((amdgpu_waves_per_eu(WAVES))) void srgemm_valu_kernel(
   if (e.gate && e.gate[tr * e.gate_ld + tc] == 0) return;
   int *flag = e.tile_flags ? &e.tile_flags[tr * tiles_c + tc] : nullptr;
   const int row0 = tr * BM, col0 = tc * BN;
-  if (FORM == FORM_FAST || (FORM == FORM_SPLIT && row0 + BM <= R && col0 + BN <= Cn))
-    valu_tile<Op, BM, BN, TM, TN, BK, false, false, FORM == FORM_SPLIT>(
-        R, Cn, K, X, ldx, Y, ldy, O, ldo, e, row0, col0, flag, sm);
-  else if (FORM == FORM_SPLIT)
+  if (!OFFGRID || (row0 + BM <= R && col0 + BN <= Cn))
+    valu_tile<Op, BM, BN, TM, TN, BK, false, false, OFFGRID>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e,
+                                                             row0, col0, flag, sm);
+  else
     valu_tile<Op, BM, BN, TM, TN, BK, false, true, true, true>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e,
                                                                row0, col0, flag, sm);
-  else
-    valu_tile<Op, BM, BN, TM, TN, BK, true>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e, row0, col0,
-                                            flag, sm);
 }
 
 // Small problems (at most four 64x64 tiles per CU; n = 1024 has one): the K
@@ -65,11 +62,10 @@ __attribute__((amdgpu_waves_per_eu(WAVES))) void srgemm_valu_kernel(
 // slabs with its own LDS buffers, and the partial tiles are combined in
 // group order, ((p0 (+) p1) (+) p2) (+) p3, before the usual epilogue: G
 // times the resident waves.  Only for the semirings whose (+) is min or max,
-// which is exact: regrouping the terms changes no bit.  CHECKED: any shape
-// and alignment, per-element bounds on loads and stores; every group runs
-// ceil(slabs / G) slabs, the ranges past K reading padding, whose terms are
-// the (+)-identity.
-template <class Op, int SK_GROUPS, bool CHECKED>
+// which is exact: regrouping the terms changes no bit.  RAGGED: any shape, as
+// OFFGRID above; every group runs ceil(slabs / G) slabs, the ranges past K
+// reading padding, whose terms are the (+)-identity.
+template <class Op, int SK_GROUPS, bool RAGGED>
 __global__ __launch_bounds__(256 * SK_GROUPS) void srgemm_valu_splitk_kernel(
     int R, int Cn, int K, const float *__restrict__ X, int64_t ldx,
     const float *__restrict__ Y, int64_t ldy, float *O, int64_t ldo, Epilogue e,
@@ -84,8 +80,12 @@ __global__ __launch_bounds__(256 * SK_GROUPS) void srgemm_valu_splitk_kernel(
   if (tid_x() == 0) sm[0].changed = 0;  // published by the main loop's barriers
   const int per = ((K + S::BK - 1) / S::BK + SK_GROUPS - 1) / SK_GROUPS;
   float acc[S::TM][S::TN];
-  valu_mainloop<Op, S::BM, S::BN, S::TM, S::TN, S::BK, CHECKED, false>(
-      R, Cn, K, X, ldx, Y, ldy, row0, col0, nullptr, 0, sm[g], acc, t, g * per, (g + 1) * per);
+  if (!RAGGED || (row0 + S::BM <= R && col0 + S::BN <= Cn))
+    valu_mainloop<Op, S::BM, S::BN, S::TM, S::TN, S::BK, false, false, RAGGED>(
+        R, Cn, K, X, ldx, Y, ldy, row0, col0, nullptr, 0, sm[g], acc, t, g * per, (g + 1) * per);
+  else
+    valu_mainloop<Op, S::BM, S::BN, S::TM, S::TN, S::BK, false, false, true, true>(
+        R, Cn, K, X, ldx, Y, ldy, row0, col0, nullptr, 0, sm[g], acc, t, g * per, (g + 1) * per);
   // The main loop ends with a barrier after every read of the slabs: groups
   // 1.. park their partial tiles in their own LDS (16 KB of its 16.5).
   static_assert(S::TM * S::TN * 256 * sizeof(float) <= sizeof(ValuSmem<S::BM, S::BN, S::BK>) -
@@ -109,13 +109,13 @@ __global__ __launch_bounds__(256 * SK_GROUPS) void srgemm_valu_splitk_kernel(
           acc[i][j] = Op::add(acc[i][j], part[(i * S::TN + j) * 256 + t]);
     }
   }
-  valu_epilogue<Op, S::BM, S::BN, S::TM, S::TN, CHECKED, false>(R, Cn, O, ldo, e, row0, col0,
-                                                                flag, &sm[0].changed, acc, t,
-                                                                g == 0);
+  valu_epilogue<Op, S::BM, S::BN, S::TM, S::TN, false, RAGGED>(R, Cn, O, ldo, e, row0, col0,
+                                                               flag, &sm[0].changed, acc, t,
+                                                               g == 0);
 }
 
-// groups > 0: the fast form (whole tiles and slab groups, aligned rows);
-// groups < 0: the checked form with -groups groups.
+// groups 4 or 2: whole tiles and slab groups; -4 or -2: the
+// ragged form of as many groups.
 template <class Op>
 hipError_t launch_splitk(int R, int Cn, int K, const float *X, int64_t ldx, const float *Y,
                          int64_t ldy, float *O, int64_t ldo, const Epilogue &e, int groups,
@@ -144,23 +144,12 @@ hipError_t launch_cfg(int R, int Cn, int K, const float *X, int64_t ldx,
   const int tiles_r = (R + Cfg::BM - 1) / Cfg::BM;
   const int tiles_c = (Cn + Cfg::BN - 1) / Cfg::BN;
   const int nthreads = (Cfg::BM / Cfg::TM) * (Cfg::BN / Cfg::TN);
-  auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  bool vec = ldx % 4 == 0 && ldy % 4 == 0 && ldo % 4 == 0 && aligned(X) && aligned(Y) &&
-             aligned(O);
-  if (e.C) vec = vec && e.ldc % 4 == 0 && aligned(e.C);
-  if (e.P) vec = vec && e.ldp % 4 == 0 && aligned(e.P);
-  const bool grid_fit = R % Cfg::BM == 0 && Cn % Cfg::BN == 0 && K % Cfg::BK == 0;
-  // the split form pays off once some tile lies wholly inside the matrix
-  const bool split = vec && R >= Cfg::BM && Cn >= Cfg::BN;
-  dim3 grid(tiles_r * tiles_c), block(nthreads);
-  if (vec && grid_fit)
-    srgemm_valu_kernel<Op, Cfg::BM, Cfg::BN, Cfg::TM, Cfg::TN, Cfg::BK, Cfg::WAVES, FORM_FAST>
-        <<<grid, block, 0, s>>>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e, tiles_r, tiles_c);
-  else if (split)
-    srgemm_valu_kernel<Op, Cfg::BM, Cfg::BN, Cfg::TM, Cfg::TN, Cfg::BK, Cfg::WAVES, FORM_SPLIT>
+  const dim3 grid(tiles_r * tiles_c), block(nthreads);
+  if (R % Cfg::BM == 0 && Cn % Cfg::BN == 0 && K % Cfg::BK == 0)
+    srgemm_valu_kernel<Op, Cfg::BM, Cfg::BN, Cfg::TM, Cfg::TN, Cfg::BK, Cfg::WAVES, false>
         <<<grid, block, 0, s>>>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e, tiles_r, tiles_c);
   else
-    srgemm_valu_kernel<Op, Cfg::BM, Cfg::BN, Cfg::TM, Cfg::TN, Cfg::BK, Cfg::WAVES, FORM_CHECKED>
+    srgemm_valu_kernel<Op, Cfg::BM, Cfg::BN, Cfg::TM, Cfg::TN, Cfg::BK, Cfg::WAVES, true>
         <<<grid, block, 0, s>>>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e, tiles_r, tiles_c);
   return hipGetLastError();
 }
@@ -195,15 +184,15 @@ ValuCfgInfo valu_cfg_info(int cfg) {
   return {CfgL::BM, CfgL::BN, CfgL::BK, 256};
 }
 
-// Tile shape choice.  Rule measured on MI355X for square problems
-// (n = 1024 .. 8192, all ops): the VALU semirings need many resident waves to
-// dual-issue, so up to ~3072^2 outputs the 64x64 tiles (7-8 waves per SIMD)
-// win; at 4096^2 the 128x64 tiles balance 2048 tiles over 1024 slots; from
-// ~6144^2 up the 128x128 tiles (fewest LDS reads per op) win.  minus_square
-// with a short K (the kNN distance step: 16384^2 x 64..128) keeps the 128x64
-// tiles at every larger area (1.38 against 1.52 ms for 128x128 and 1.53 for
-// 64x64 at 16384^2 x 128).  Shapes the autotuner has timed (simd2_autotune)
-// use the recorded winner instead.
+// Tile shape choice, measured on MI355X for square problems (n = 1024 .. 8192,
+// min_plus / max_min / minus_square, us in 64x64, 128x64 and 128x128 tiles for
+// min_plus): the 64x64 tiles' many workgroups waste least of a last round
+// (3328: 965, 1058, 1181; 4608: 2451, 2570, 2891; 5120: 3260, 3337, 3663; 7168:
+// 8788, 8782, 9090); the 128x128 tiles read LDS least and win where their own
+// rounds fill (6144: 5558, 5407, 5479, three rounds; 8192: 12893, 12620,
+// 12588; minus_square 16384^2 x 128: 1432, 1384, 1310).  At 4096 all three
+// agree within 2% and the 128x64 tiles, two full rounds, are kept.  Shapes the
+// autotuner has timed (simd2_autotune) use the recorded winner instead.
 namespace {
 struct TunedEntry { int op, R, Cn, K, cfg; };
 constexpr int TUNED_MAX = 64;
@@ -233,36 +222,23 @@ int valu_pick_cfg(int op, int R, int Cn, int K) {
   const double area = (double)R * Cn;
   const double scale = 256.0 / device_cu_count();   // rule is for 256 CUs
   const double a = area * scale;
-  if (a <= 3072.0 * 3072.0 * 1.01) return CFG_S64;
-  if (a <= 4096.0 * 4096.0 * 1.01) return CFG_M128x64;
-  if (op == 8 && K <= 128) return CFG_M128x64;
-  return CFG_L128;
+  if (a <= 4096.0 * 4096.0 * 1.01) return a > 3840.0 * 3840.0 ? CFG_M128x64 : CFG_S64;
+  const double rounds = (double)((R + 127) / 128) * ((Cn + 127) / 128) / (3 * device_cu_count());
+  return a >= 5900.0 * 5900.0 && rounds >= 0.85 * ceil(rounds) ? CFG_L128 : CFG_S64;
 }
 
-// The split-K form (automatic choice only): a min/max semiring, the 64x64
-// tiles chosen, at most four tiles per CU, no gate.  Returns the group count
-// G for the fast form (a whole number of tiles and of G-slab groups, every
-// operand 16-byte aligned row by row), -G for the checked form (operands
-// whose rows are not all 16-byte aligned, where the unsplit kernel takes its
-// checked body too, and aligned off-grid shapes of at most two tiles per CU,
-// where four groups' waves outweigh the unsplit kernel's 128-bit interior
-// loads: 1000x776x300 min_plus 39 -> 31 us), 0 when the split does not apply.
-static int splitk_groups(int op, int R, int Cn, int K, const float *X, int64_t ldx,
-                         const float *Y, int64_t ldy, const float *O, int64_t ldo,
-                         const Epilogue &e) {
+// How a min / max semiring splits K where the 64x64 tiles were chosen and are
+// few: 4 / 2 groups of 256 threads, up to two / four tiles per CU, negative off
+// the grid (1025x1023x1021 77 us; 1999x1801x777 104, 111 unsplit); 0 -- unsplit.
+static int splitk_groups(int op, int R, int Cn, int K, const Epilogue &e) {
   if (op == 1 || op == 8 || op < 0 || op > 6 || e.gate || K <= 0) return 0;
   const int64_t tiles =
       (int64_t)((R + CfgS::BM - 1) / CfgS::BM) * ((Cn + CfgS::BN - 1) / CfgS::BN);
-  const int groups = tiles < 2 * device_cu_count() ? 4 : tiles <= 4 * device_cu_count() ? 2 : 0;
+  const int64_t cus = device_cu_count();
+  const int groups = tiles < 2 * cus ? 4 : tiles <= 4 * cus ? 2 : 0;
   if (groups == 0) return 0;
-  auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-  bool vec = ldx % 4 == 0 && ldy % 4 == 0 && ldo % 4 == 0 && aligned(X) && aligned(Y) &&
-             aligned(O);
-  if (e.C) vec = vec && e.ldc % 4 == 0 && aligned(e.C);
-  if (e.P) vec = vec && e.ldp % 4 == 0 && aligned(e.P);
-  if (!vec) return -groups;
   if (R % CfgS::BM == 0 && Cn % CfgS::BN == 0 && K % (CfgS::BK * groups) == 0) return groups;
-  return groups == 4 ? -4 : 0;
+  return -groups;
 }
 
 hipError_t launch_valu_f32(int op, int R, int Cn, int K, const float *X,
@@ -271,7 +247,7 @@ hipError_t launch_valu_f32(int op, int R, int Cn, int K, const float *X,
                            int cfg) {
   if (cfg == CFG_AUTO) {
     cfg = valu_pick_cfg(op, R, Cn, K);
-    const int g = cfg == CFG_S64 ? splitk_groups(op, R, Cn, K, X, ldx, Y, ldy, O, ldo, e) : 0;
+    const int g = cfg == CFG_S64 ? splitk_groups(op, R, Cn, K, e) : 0;
     if (g) {
       switch (op) {
       case 0: return launch_splitk<MinPlus>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e, g, s);

@@ -18,6 +18,10 @@ constexpr int NUM_XCD = 8;
 // struct is copied with memcpy, which scalar replacement does not always
 // undo, and the staged slab then lives in scratch.
 typedef float vf4 __attribute__((ext_vector_type(4)));
+// The same in memory, at any 4-byte alignment: global loads and stores of 16
+// bytes need no more on this hardware, so rows of any leading dimension move
+// 16 bytes a lane (min_plus 1025x1023x1021 110 us element by element).
+typedef float vf4u __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ void map_tile(int b, int tiles_r, int tiles_c,
                                          int &tr, int &tc) {
@@ -93,7 +97,7 @@ __device__ __forceinline__ void load_slab_form(vf4 (&xv)[BM * BK / 4 / NT],
       if (GUARD && r >= R)
         xv[h] = vf4{Op::pad_x, Op::pad_x, Op::pad_x, Op::pad_x};
       else
-        xv[h] = *reinterpret_cast<const vf4 *>(X + (int64_t)r * ldx + k);
+        xv[h] = *reinterpret_cast<const vf4u *>(X + (int64_t)r * ldx + k);
     } else {
       float t[4];
 #pragma unroll
@@ -114,7 +118,7 @@ __device__ __forceinline__ void load_slab_form(vf4 (&xv)[BM * BK / 4 / NT],
         for (int q = 0; q < 4; ++q) t[q] = c + q < Cn ? Y[(int64_t)k * ldy + c + q] : Op::pad_y;
         yv[h] = vf4{t[0], t[1], t[2], t[3]};
       } else {
-        yv[h] = *reinterpret_cast<const vf4 *>(Y + (int64_t)k * ldy + c);
+        yv[h] = *reinterpret_cast<const vf4u *>(Y + (int64_t)k * ldy + c);
       }
     } else {
       float t[4];
@@ -332,7 +336,7 @@ __device__ __forceinline__ void valu_epilogue(int R, int Cn, float *O, int64_t l
         for (int q = 0; q < 4; ++q) v[q] = acc[i][gj * 4 + q];
         if (!CHECKED && (!MASKED || (r < R && c + 4 <= Cn))) {
           if (e.C) {
-            const float4 cv = *reinterpret_cast<const float4 *>(e.C + (int64_t)r * e.ldc + c);
+            const vf4u cv = *reinterpret_cast<const vf4u *>(e.C + (int64_t)r * e.ldc + c);
             v[0] = Op::add(v[0], cv.x); v[1] = Op::add(v[1], cv.y);
             v[2] = Op::add(v[2], cv.z); v[3] = Op::add(v[3], cv.w);
           }
@@ -341,11 +345,11 @@ __device__ __forceinline__ void valu_epilogue(int R, int Cn, float *O, int64_t l
             for (int q = 0; q < 4; ++q) v[q] = (v[q] > -1.0f && v[q] < 1.0f) ? -FLT_MAX : v[q];
           }
           if (e.P) {
-            const float4 pv = *reinterpret_cast<const float4 *>(e.P + (int64_t)r * e.ldp + c);
+            const vf4u pv = *reinterpret_cast<const vf4u *>(e.P + (int64_t)r * e.ldp + c);
             changed |= differs(v[0], pv.x, e.mode) | differs(v[1], pv.y, e.mode) |
                        differs(v[2], pv.z, e.mode) | differs(v[3], pv.w, e.mode);
           }
-          *reinterpret_cast<float4 *>(O + (int64_t)r * ldo + c) = make_float4(v[0], v[1], v[2], v[3]);
+          *reinterpret_cast<vf4u *>(O + (int64_t)r * ldo + c) = vf4u{v[0], v[1], v[2], v[3]};
         } else {
           if (r < R) {
 #pragma unroll
