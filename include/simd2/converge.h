@@ -44,7 +44,8 @@ enum {
    * device-to-host flag read (apps/apsp/cuASR/apsp_cuASR.cu:42-54). */
   SIMD2_CONVERGE_REFERENCE = 0,
   /* Change test fused into the squaring's epilogue, X and work swap roles
-   * each iteration; one 4-byte flag read per iteration. */
+   * each iteration; several squarings are enqueued per 4-byte flag read (one
+   * behind a squaring that changed nothing is skipped on the device). */
   SIMD2_CONVERGE_FUSED = 1
 };
 
@@ -55,7 +56,8 @@ enum {
  * On return X holds the result and *num_itr the number of squarings,
  * counting the final one that changed nothing, as the reference counts it.
  * Returns SIMD2_ERROR_NOT_CONVERGED if the cap was hit while X still
- * changed.  Blocks the calling thread (one flag read per squaring). */
+ * changed.  *flag_d is scratch.  Blocks the calling thread until X holds the
+ * result. */
 int simd2_converge_f32(int op, int n, float *X, int ldx, float *work, int ldw,
                        int *flag_d, int do_epilogue, int check_mode,
                        int max_itr, int flags, hipStream_t stream,

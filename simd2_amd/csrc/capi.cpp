@@ -84,6 +84,50 @@ int srgemm_i32_cm(int M, int N, int K, const int *A, int lda, const int *B, int 
                                      ldc, nullptr, 0, nullptr, s));
 }
 
+int read_flag(int *flag_d, hipStream_t s, int *out) {
+  int h = 0;
+  hipError_t e = hipMemcpyAsync(&h, flag_d, sizeof(int), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  *out = h;
+  return hip_status(e);
+}
+
+// The fused loops' driver.  square(step) enqueues squaring `step` (1, 2, ...),
+// which raises *flag_d to `step` when it changes something and is skipped on
+// the device when the one before it changed nothing (FlagStep), so several are
+// enqueued per look at the flag: a look costs a copy, a synchronisation and a
+// GPU that has gone idle (20 us, and at n = 1024 the next squaring 10 us more),
+// a skipped squaring 1 us while the host is waiting anyway.  Two first, so that
+// a matrix that is closed already pays nothing for the second (95 -> 96 us at
+// n = 1024; six first: 124), then four at a time; more than five in a row
+// without a wait cost 20 us by themselves.  min_plus, one look per squaring ->
+// here, by squarings needed: n = 64: 2: 70 -> 49 us, 4: 127 -> 85, 7: 226 ->
+// 139; n = 1024: 138 -> 116, 262 -> 220, 467 -> 379.  *itr: the squarings that
+// ran, the last of which changed nothing unless *run.
+template <class Square>
+int converge_ahead(int *flag_d, int max_itr, hipStream_t stream, Square &&square, int *itr,
+                   int *run) {
+  constexpr int FIRST = 2, NEXT = 4;
+  int enqueued = 0, last = 0;
+  *itr = 0;
+  *run = 1;
+  while (*run && enqueued < max_itr) {
+    const int upto = std::min(max_itr, enqueued + (enqueued ? NEXT : FIRST));
+    while (enqueued < upto) {
+      const hipError_t e = square(++enqueued);
+      if (e != hipSuccess) {
+        *itr = enqueued;
+        return hip_status(e);
+      }
+    }
+    const int st = read_flag(flag_d, stream, &last);
+    *run = last >= enqueued;
+    *itr = *run ? enqueued : last + 1;
+    if (st != SIMD2_SUCCESS) return st;
+  }
+  return SIMD2_SUCCESS;
+}
+
 }  // namespace
 
 extern "C" {
@@ -215,7 +259,7 @@ int simd2_orand_packed(int M, int N, int K, const uint32_t *A, int lda_words,
   }
   return hip_status(launch_orand_packed(M, N, K, A, lda_words, B, ldb_words,
                                         do_epilogue ? C : nullptr, ldc_words, D, ldd_words,
-                                        nullptr, 0, nullptr, stream));
+                                        nullptr, 0, FlagStep{}, stream));
 }
 
 size_t simd2_minus_square_workspace(int M, int N, int K) {
@@ -345,14 +389,6 @@ bool comp_update_int(int *prev, int *cur, int *check, int *check_h, int M, int N
   return comp_update_common(prev, cur, check, check_h, M, N, 0, true);
 }
 
-static int read_flag(int *flag_d, hipStream_t s, int *out) {
-  int h = 0;
-  hipError_t e = hipMemcpyAsync(&h, flag_d, sizeof(int), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  *out = h;
-  return hip_status(e);
-}
-
 int simd2_converge_f32(int op, int n, float *X, int ldx, float *work, int ldw, int *flag_d,
                        int do_epilogue, int check_mode, int max_itr, int flags,
                        hipStream_t stream, int *num_itr) {
@@ -367,49 +403,62 @@ int simd2_converge_f32(int op, int n, float *X, int ldx, float *work, int ldw, i
   if (!X || !work || !flag_d) return SIMD2_ERROR_NULL_POINTER;
   if (overlap(span(X, n, n, ldx, 4), span(work, n, n, ldw, 4))) return SIMD2_ERROR_ALIASING;
 
-  float *cur = X, *nxt = work;
-  int64_t ldcur = ldx, ldnxt = ldw;
   int itr = 0, run = 1;
   hipError_t e = hipSuccess;
+  if (flags == SIMD2_CONVERGE_FUSED) {
+    e = launch_fill_i32(flag_d, 0, 1, stream);
+    if (e != hipSuccess) return hip_status(e);
+    // odd squarings read X and write work, even ones the other way round
+    const int st = converge_ahead(flag_d, max_itr, stream, [&](int step) {
+      float *from = step & 1 ? X : work, *to = step & 1 ? work : X;
+      const int64_t ldf = step & 1 ? ldx : ldw, ldt = step & 1 ? ldw : ldx;
+      Epilogue ep;
+      if (do_epilogue) {
+        ep.C = from;
+        ep.ldc = ldf;
+      }
+      ep.P = from;
+      ep.ldp = ldf;
+      ep.flag = flag_d;
+      ep.step = step;
+      ep.mode = check_mode;
+      return launch_valu_f32(op, n, n, n, from, ldf, from, ldf, to, ldt, ep, stream);
+    }, &itr, &run);
+    if (num_itr) *num_itr = itr;
+    if (st != SIMD2_SUCCESS) return st;
+    if (itr & 1) {
+      e = launch_copy_2d(X, (int64_t)ldx * 4, work, (int64_t)ldw * 4, n, n * 4, stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(stream);
+      if (e != hipSuccess) return hip_status(e);
+    }
+    return run ? SIMD2_ERROR_NOT_CONVERGED : SIMD2_SUCCESS;
+  }
   while (run && itr < max_itr) {
     ++itr;
     e = launch_fill_i32(flag_d, 0, 1, stream);
     if (e != hipSuccess) break;
     Epilogue ep;
     if (do_epilogue) {
-      ep.C = cur;
-      ep.ldc = ldcur;
+      ep.C = X;
+      ep.ldc = ldx;
     }
-    if (flags == SIMD2_CONVERGE_FUSED) {
-      ep.P = cur;
-      ep.ldp = ldcur;
-      ep.flag = flag_d;
-      ep.mode = check_mode;
-      e = launch_valu_f32(op, n, n, n, cur, ldcur, cur, ldcur, nxt, ldnxt, ep, stream);
-      if (e != hipSuccess) break;
-      std::swap(cur, nxt);
-      std::swap(ldcur, ldnxt);
+    e = launch_valu_f32(op, n, n, n, X, ldx, X, ldx, work, ldw, ep, stream);
+    if (e != hipSuccess) break;
+    if (ldx == n && ldw == n) {
+      e = launch_comp_update_f32(X, work, flag_d, (int64_t)n * n, check_mode, stream);
     } else {
-      e = launch_valu_f32(op, n, n, n, cur, ldcur, cur, ldcur, nxt, ldnxt, ep, stream);
-      if (e != hipSuccess) break;
-      if (ldcur == n && ldnxt == n) {
-        e = launch_comp_update_f32(cur, nxt, flag_d, (int64_t)n * n, check_mode, stream);
-      } else {
-        // strided matrices: compare row by row through the same kernel
-        for (int r = 0; r < n && e == hipSuccess; ++r)
-          e = launch_comp_update_f32(cur + (int64_t)r * ldcur, nxt + (int64_t)r * ldnxt, flag_d,
-                                     n, check_mode, stream);
-      }
-      if (e != hipSuccess) break;
+      // strided matrices: compare row by row through the same kernel
+      for (int r = 0; r < n && e == hipSuccess; ++r)
+        e = launch_comp_update_f32(X + (int64_t)r * ldx, work + (int64_t)r * ldw, flag_d, n,
+                                   check_mode, stream);
     }
+    if (e != hipSuccess) break;
     const int st = read_flag(flag_d, stream, &run);
     if (st != SIMD2_SUCCESS) {
       if (num_itr) *num_itr = itr;
       return st;
     }
   }
-  if (e == hipSuccess && cur != X)
-    e = launch_copy_2d(X, (int64_t)ldx * 4, cur, ldcur * 4, n, n * 4, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
   if (num_itr) *num_itr = itr;
   if (e != hipSuccess) return hip_status(e);
@@ -437,26 +486,19 @@ int simd2_converge_i32(int n, int *X, int ldx, int *work, int ldw, int *flag_d, 
   // into X.
   if (flags == SIMD2_CONVERGE_FUSED && n >= 64 && max_itr > 0) {
     const int nw = (n + 31) / 32;
-    uint32_t *pc = reinterpret_cast<uint32_t *>(work), *pn = pc + nw;
+    uint32_t *p0 = reinterpret_cast<uint32_t *>(work), *p1 = p0 + nw;
     e = launch_fill_i32(flag_d, 0, 1, stream);
-    if (e == hipSuccess) e = launch_pack_i32(n, n, X, ldx, pc, ldw, flag_d, stream);
-    while (e == hipSuccess && run && itr < max_itr) {
-      ++itr;
-      if (itr > 1) e = launch_fill_i32(flag_d, 0, 1, stream);
-      if (e == hipSuccess)
-        e = launch_orand_packed(n, n, n, pc, ldw, pc, ldw, pc, ldw, pn, ldw, pc, ldw, flag_d,
-                                stream);
-      if (e != hipSuccess) break;
-      std::swap(pc, pn);
-      const int st = read_flag(flag_d, stream, &run);
-      if (st != SIMD2_SUCCESS) {
-        if (num_itr) *num_itr = itr;
-        return st;
-      }
-    }
-    if (e == hipSuccess) e = launch_unpack_i32(n, n, pc, ldw, X, ldx, stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    if (e == hipSuccess) e = launch_pack_i32(n, n, X, ldx, p0, ldw, flag_d, stream);
+    if (e != hipSuccess) return hip_status(e);
+    const int st = converge_ahead(flag_d, max_itr, stream, [&](int step) {
+      uint32_t *from = step & 1 ? p0 : p1, *to = step & 1 ? p1 : p0;
+      return launch_orand_packed(n, n, n, from, ldw, from, ldw, from, ldw, to, ldw, from, ldw,
+                                 FlagStep{flag_d, step}, stream);
+    }, &itr, &run);
     if (num_itr) *num_itr = itr;
+    if (st != SIMD2_SUCCESS) return st;
+    e = launch_unpack_i32(n, n, itr & 1 ? p1 : p0, ldw, X, ldx, stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(stream);
     if (e != hipSuccess) return hip_status(e);
     return run ? SIMD2_ERROR_NOT_CONVERGED : SIMD2_SUCCESS;
   }
@@ -508,30 +550,22 @@ int simd2_converge_orand_packed(int n, uint32_t *X, int ldx_words, uint32_t *wor
   if (!X || !work || !flag_d) return SIMD2_ERROR_NULL_POINTER;
   if (overlap(span(X, nw, n, ldx_words, 4), span(work, nw, n, ldw_words, 4)))
     return SIMD2_ERROR_ALIASING;
-  uint32_t *cur = X, *nxt = work;
-  int64_t ldcur = ldx_words, ldnxt = ldw_words;
   int itr = 0, run = 1;
-  hipError_t e = hipSuccess;
-  while (run && itr < max_itr) {
-    ++itr;
-    e = launch_fill_i32(flag_d, 0, 1, stream);
-    if (e != hipSuccess) break;
-    e = launch_orand_packed(n, n, n, cur, ldcur, cur, ldcur, cur, ldcur, nxt, ldnxt, cur, ldcur,
-                            flag_d, stream);
-    if (e != hipSuccess) break;
-    std::swap(cur, nxt);
-    std::swap(ldcur, ldnxt);
-    const int st = read_flag(flag_d, stream, &run);
-    if (st != SIMD2_SUCCESS) {
-      if (num_itr) *num_itr = itr;
-      return st;
-    }
-  }
-  if (e == hipSuccess && cur != X)
-    e = launch_copy_2d(X, (int64_t)ldx_words * 4, cur, ldcur * 4, n, nw * 4, stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  if (num_itr) *num_itr = itr;
+  hipError_t e = launch_fill_i32(flag_d, 0, 1, stream);
   if (e != hipSuccess) return hip_status(e);
+  const int st = converge_ahead(flag_d, max_itr, stream, [&](int step) {
+    uint32_t *from = step & 1 ? X : work, *to = step & 1 ? work : X;
+    const int64_t ldf = step & 1 ? ldx_words : ldw_words, ldt = step & 1 ? ldw_words : ldx_words;
+    return launch_orand_packed(n, n, n, from, ldf, from, ldf, from, ldf, to, ldt, from, ldf,
+                               FlagStep{flag_d, step}, stream);
+  }, &itr, &run);
+  if (num_itr) *num_itr = itr;
+  if (st != SIMD2_SUCCESS) return st;
+  if (itr & 1) {
+    e = launch_copy_2d(X, (int64_t)ldx_words * 4, work, (int64_t)ldw_words * 4, n, nw * 4, stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    if (e != hipSuccess) return hip_status(e);
+  }
   return run ? SIMD2_ERROR_NOT_CONVERGED : SIMD2_SUCCESS;
 }
 

@@ -26,6 +26,20 @@ struct Epilogue {
                              // 2 APLP: o in (-1,1) -> -FLT_MAX, then o != p
   const int *gate = nullptr; // when set, tile (tr, tc) is computed only if
   int gate_ld = 0;           //   gate[tr * gate_ld + tc] != 0
+  int step = 1;              // *flag becomes max(*flag, step) when any element
+                             //   changed, and nothing is computed while *flag
+                             //   < step - 1: see FlagStep
+};
+
+// Squarings enqueued ahead of the host's look at the change flag.  Squaring
+// `step` (1, 2, ...) raises *flag to `step` when it changes something, and is
+// skipped as a whole, its output untouched, when *flag < step - 1: a squaring
+// before it changed nothing.  So *flag counts the squarings that changed
+// something, whatever number was enqueued behind them.  step 1 (with *flag
+// cleared) is a plain 0 / 1 flag.
+struct FlagStep {
+  int *flag = nullptr;
+  int step = 1;
 };
 
 enum CheckMode { CHECK_EXACT = 0, CHECK_THRESHOLD = 1, CHECK_APLP = 2 };
@@ -93,7 +107,7 @@ hipError_t launch_orand_packed(int M, int N, int K, const uint32_t *A,
                                int64_t lda, const uint32_t *B, int64_t ldb,
                                const uint32_t *C, int64_t ldc, uint32_t *D,
                                int64_t ldd, const uint32_t *P, int64_t ldp,
-                               int *flag, hipStream_t s);
+                               FlagStep flag, hipStream_t s);
 
 // FP16-input emulation kernel and conversions (tensor_emu.hip).
 hipError_t launch_tensor_emu(int op, const void *a, const void *b, const float *c, float *d,

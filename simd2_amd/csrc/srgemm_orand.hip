@@ -43,6 +43,11 @@ __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t b, uint32_t acc)
   return r;
 }
 
+// Whether this launch belongs to a squaring behind one that changed nothing.
+__device__ __forceinline__ bool flag_done(const FlagStep &f) {
+  return f.flag && f.step > 1 && *f.flag < f.step - 1;
+}
+
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
@@ -101,7 +106,7 @@ template <int MB, int NB, int WR, int WC> struct OrandCfg {
 template <int MB, int NB, int WR, int WC, bool VEC>
 __global__ __launch_bounds__(WR * WC * 64) void orand_packed_kernel(
     int M, int NW, int K, const uint32_t *__restrict__ A, uint32_t lda, OrandB B, const uint32_t *C,
-    int64_t ldc, uint32_t *D, int64_t ldd, const uint32_t *P, int64_t ldp, int *flag,
+    int64_t ldc, uint32_t *D, int64_t ldd, const uint32_t *P, int64_t ldp, FlagStep flag,
     uint32_t last_mask, int tiles_c, int ksplit, int kw_per) {
   using Cfg = OrandCfg<MB, NB, WR, WC>;
   constexpr int BM = Cfg::BM, NT = Cfg::NT, WPT = Cfg::WPT;
@@ -113,6 +118,7 @@ __global__ __launch_bounds__(WR * WC * 64) void orand_packed_kernel(
   // bit 2 rb + h: A rows 32 rb.. hold a 1 in 64-k half h; bit 16 + 2 cb + h:
   // the same for B columns 32 cb..
   __shared__ uint32_t some[3];
+  if (flag_done(flag)) return;
   const int tid = tid_x();
   const int lane = tid % 64;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -306,9 +312,9 @@ __global__ __launch_bounds__(WR * WC * 64) void orand_packed_kernel(
       }
     }
   }
-  if (flag && ksplit == 1) {
+  if (flag.flag && ksplit == 1) {
     const bool any = __any(changed);
-    if (any && lane == 0) atomicOr(flag, 1);
+    if (any && lane == 0) atomicMax(flag.flag, flag.step);
   }
 }
 
@@ -318,7 +324,8 @@ using OrandS = OrandCfg<2, 2, 2, 2>;  // 128x128, 4 waves
 // D = C (or zero), last word masked: the start of a K-split product.
 __global__ __launch_bounds__(256) void orand_init_kernel(int M, int NW, const uint32_t *C,
                                                          int64_t ldc, uint32_t *D, int64_t ldd,
-                                                         uint32_t last_mask) {
+                                                         uint32_t last_mask, FlagStep flag) {
+  if (flag_done(flag)) return;
   const int64_t total = (int64_t)M * NW;
   for (int64_t e = (int64_t)bid_x() * 256 + tid_x(); e < total; e += (int64_t)gridDim.x * 256) {
     const int r = (int)(e / NW), w = (int)(e % NW);
@@ -333,7 +340,8 @@ __global__ __launch_bounds__(256) void orand_init_kernel(int M, int NW, const ui
 __global__ __launch_bounds__(256) void orand_diff_kernel(int M, int NW, const uint32_t *D,
                                                          int64_t ldd, const uint32_t *P,
                                                          int64_t ldp, uint32_t last_mask,
-                                                         int *flag) {
+                                                         FlagStep flag) {
+  if (flag_done(flag)) return;
   const int64_t total = (int64_t)M * NW;
   bool changed = false;
   for (int64_t e = (int64_t)bid_x() * 256 + tid_x(); e < total; e += (int64_t)gridDim.x * 256) {
@@ -341,7 +349,7 @@ __global__ __launch_bounds__(256) void orand_diff_kernel(int M, int NW, const ui
     const uint32_t m = w == NW - 1 ? last_mask : ~0u;
     changed |= (D[(int64_t)r * ldd + w] & m) != (P[(int64_t)r * ldp + w] & m);
   }
-  if (__syncthreads_or(changed) && tid_x() == 0) atomicOr(flag, 1);
+  if (__syncthreads_or(changed) && tid_x() == 0) atomicMax(flag.flag, flag.step);
 }
 
 // ---- int32 booleans -------------------------------------------------------
@@ -458,7 +466,7 @@ namespace {
 template <class Cfg, bool VEC, int MB, int NB, int WR, int WC>
 void launch_orand_tiles(OrandCfg<MB, NB, WR, WC>, int M, int NW, int K, const uint32_t *A,
                         int64_t lda, const OrandB &B, const uint32_t *C, int64_t ldc, uint32_t *D,
-                        int64_t ldd, const uint32_t *P, int64_t ldp, int *flag,
+                        int64_t ldd, const uint32_t *P, int64_t ldp, FlagStep flag,
                         uint32_t last_mask, int ksplit, int kw_per, hipStream_t s) {
   const int tiles_r = (M + Cfg::BM - 1) / Cfg::BM;
   const int tiles_c = (NW + Cfg::BM / 32 - 1) / (Cfg::BM / 32);
@@ -471,7 +479,7 @@ void launch_orand_tiles(OrandCfg<MB, NB, WR, WC>, int M, int NW, int K, const ui
 // the words past K and N).
 hipError_t launch_orand_rows(int M, int N, int K, const uint32_t *A, int64_t lda, const OrandB &B,
                              bool padded, const uint32_t *C, int64_t ldc, uint32_t *D, int64_t ldd,
-                             const uint32_t *P, int64_t ldp, int *flag, hipStream_t s) {
+                             const uint32_t *P, int64_t ldp, FlagStep flag, hipStream_t s) {
   const int NW = (N + 31) / 32;
   if (M <= 0 || NW <= 0) return hipSuccess;
   const uint32_t last_mask = (N & 31) ? ((1u << (N & 31)) - 1u) : ~0u;
@@ -492,7 +500,7 @@ hipError_t launch_orand_rows(int M, int N, int K, const uint32_t *A, int64_t lda
   const int64_t words = (int64_t)M * NW;
   const int egrid = (int)std::min<int64_t>((words + 255) / 256, 2048);
   if (ksplit > 1)
-    orand_init_kernel<<<dim3(egrid), dim3(256), 0, s>>>(M, NW, C, ldc, D, ldd, last_mask);
+    orand_init_kernel<<<dim3(egrid), dim3(256), 0, s>>>(M, NW, C, ldc, D, ldd, last_mask, flag);
   auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   // 16-byte loads read whole groups of four words: rows must hold them
   const bool vec = aligned(A) && aligned(B.p) && lda % 4 == 0 && B.ld % 4 == 0 &&
@@ -509,7 +517,7 @@ hipError_t launch_orand_rows(int M, int N, int K, const uint32_t *A, int64_t lda
   else
     launch_orand_tiles<OrandS, false>(OrandS{}, M, NW, K, A, lda, B, C, ldc, D, ldd, P, ldp, flag,
                                       last_mask, ksplit, kw_per, s);
-  if (ksplit > 1 && P && flag)
+  if (ksplit > 1 && P && flag.flag)
     orand_diff_kernel<<<dim3(egrid), dim3(256), 0, s>>>(M, NW, D, ldd, P, ldp, last_mask, flag);
   return hipGetLastError();
 }
@@ -684,7 +692,7 @@ hipError_t launch_orand_packed(int M, int N, int K, const uint32_t *A,
                                int64_t lda, const uint32_t *B, int64_t ldb,
                                const uint32_t *C, int64_t ldc, uint32_t *D,
                                int64_t ldd, const uint32_t *P, int64_t ldp,
-                               int *flag, hipStream_t s) {
+                               FlagStep flag, hipStream_t s) {
   return launch_orand_rows(M, N, K, A, lda, OrandB{B, (uint32_t)ldb, 0, -1, 31}, false, C, ldc, D, ldd, P, ldp,
                            flag, s);
 }
@@ -767,7 +775,7 @@ bool orand_i32_packed(int R, int Cn, int K, const int *X, int64_t ldx, const int
     if (e == hipSuccess)
       e = launch_orand_rows(R, Cn, k, px, ldo,
                             OrandB{py, (uint32_t)ldo, (uint32_t)nwp, jy.mask, shift}, true,
-                            C || k0 > 0 ? res : nullptr, ldo, res, ldo, nullptr, 0, nullptr, s);
+                            C || k0 > 0 ? res : nullptr, ldo, res, ldo, nullptr, 0, FlagStep{}, s);
   }
   if (e == hipSuccess) e = launch_unpack_i32(R, Cn, res, ldo, O, ldo, s);
   *status = e;

@@ -43,6 +43,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES))) void srgemm_valu_kernel(
     const float *__restrict__ Y, int64_t ldy, float *O, int64_t ldo,
     Epilogue e, int tiles_r, int tiles_c) {
   __shared__ ValuSmem<BM, BN, BK> sm;
+  if (flag_done(e.flag, e.step)) return;
   int tr, tc;
   map_tile(bid_x(), tiles_r, tiles_c, tr, tc);
   if (e.gate && e.gate[tr * e.gate_ld + tc] == 0) return;
@@ -72,6 +73,7 @@ __global__ __launch_bounds__(256 * SK_GROUPS) void srgemm_valu_splitk_kernel(
     int tiles_r, int tiles_c) {
   using S = CfgS;
   __shared__ ValuSmem<S::BM, S::BN, S::BK> sm[SK_GROUPS];
+  if (flag_done(e.flag, e.step)) return;
   int tr, tc;
   map_tile(bid_x(), tiles_r, tiles_c, tr, tc);
   int *flag = e.tile_flags ? &e.tile_flags[tr * tiles_c + tc] : nullptr;

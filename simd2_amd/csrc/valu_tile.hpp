@@ -48,6 +48,11 @@ __device__ __forceinline__ bool differs(float o, float p, int mode) {
   return bits;
 }
 
+// Whether this launch is a squaring behind one that changed nothing.
+__device__ __forceinline__ bool flag_done(const int *flag, int step) {
+  return flag && step > 1 && *flag < step - 1;
+}
+
 // Load one BK-deep slab of X (BM x BK, k contiguous) and Y (BK x BN) into
 // registers.  Fast path: 128-bit loads; checked path: per-element bounds
 // with the op's padding values.
@@ -370,7 +375,7 @@ __device__ __forceinline__ void valu_epilogue(int R, int Cn, float *O, int64_t l
   }
   if (e.flag || tile_flag) {
     const bool any = __any(changed);
-    if (e.flag && any && (tid % warpSize) == 0) atomicOr(e.flag, 1);
+    if (e.flag && any && (tid % warpSize) == 0) atomicMax(e.flag, e.step);
     if (tile_flag) {
       if (any && (tid % warpSize) == 0) atomicOr(changed_slot, 1);
       __syncthreads();

@@ -158,3 +158,43 @@ def test_closure_i32_any_values_and_stride(gpu, oracle_mod, n):
             assert st == (0 if max_itr == 500 else simd2_amd.ERROR_NOT_CONVERGED)
             assert np.array_equal(X.cpu().numpy(), want), (flags, max_itr)
             assert bool((wide[:, n:] == 5).all()), "wrote past the row"
+
+
+# Squarings are enqueued 2, then 4 at a time: caps and convergence on both
+# sides of each look at the flag, and with an odd and an even last squaring
+# (the result lies in the work matrix or in X).  n = 48 takes the int32 loop
+# that isn't packed; 64 and 1100 also the split and the one-pass products.
+@pytest.mark.parametrize("kind", ["min_plus", "threshold", "int32", "packed"])
+@pytest.mark.parametrize("n", [48, 64, 1100])
+def test_looks_at_the_flag(gpu, kind, n):
+    import simd2_amd
+    torch = gpu
+    for edges in (1, 2, 4, 5, 16, 33):  # 1, 2, 3, 4, 5 and 7 squarings
+        needed = int(np.ceil(np.log2(edges))) + 1
+        for cap in (0, 1, 2, 3, 5, 6, 7, 10):
+            ran = min(cap, needed)
+            hops = 1 << ran
+            d = np.arange(n)[None, :] - np.arange(n)[:, None]
+            on_path = (np.arange(n)[None, :] <= edges) & (np.arange(n)[:, None] <= edges)
+            far = (d >= 0) & ((d == 0) | (on_path & (d <= hops)))
+            near = (d >= 0) & ((d == 0) | (on_path & (d <= 1)))
+            if kind in ("min_plus", "threshold"):
+                X0 = torch.from_numpy(np.where(near, d, np.inf).astype(np.float32)).cuda()
+                want = np.where(far, d, np.inf).astype(np.float32)
+                wide = torch.full((n, n + 3), 7.0, device="cuda")
+                X = wide[:, :n].copy_(X0) if n == 64 else X0
+                X, itr, st = simd2_amd.converge(
+                    "min_plus", X, check="exact" if kind == "min_plus" else "threshold",
+                    max_itr=cap, work=torch.full((n, n), 5.0, device="cuda"))
+            else:
+                X0 = torch.from_numpy(near.astype(np.int32)).cuda()
+                want = far.astype(np.int32)
+                if kind == "int32":
+                    X, itr, st = simd2_amd.converge("or_and", X0, max_itr=cap)
+                else:
+                    P, itr, st = simd2_amd.converge("or_and", simd2_amd.pack_bits(X0),
+                                                    max_itr=cap)
+                    X = simd2_amd.unpack_bits(P, n)
+            assert itr == ran, (edges, cap)
+            assert st == (0 if cap >= needed else simd2_amd.ERROR_NOT_CONVERGED), (edges, cap)
+            assert np.array_equal(X.cpu().numpy(), want), (edges, cap)
