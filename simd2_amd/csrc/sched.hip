@@ -53,6 +53,7 @@ __attribute__((amdgpu_waves_per_eu(G > 1 ? 1 : Cfg::WAVES))) void sched_kernel(S
   __shared__ int s_cnt;
   __shared__ int s_wave[4];
   __shared__ unsigned s_bits[2];
+  __shared__ int s_chg[2];
 
   // A squaring after one that changed nothing computes nothing: the result
   // stays where that squaring left it.
@@ -72,6 +73,8 @@ __attribute__((amdgpu_waves_per_eu(G > 1 ? 1 : Cfg::WAVES))) void sched_kernel(S
     s_cnt = 0;
     s_bits[0] = 0;
     s_bits[1] = 0;
+    s_chg[0] = 0;
+    s_chg[1] = 0;
   }
   __syncthreads();
   const uint8_t *xo = a.xocc_in + (int64_t)tr * a.slabs;
@@ -186,12 +189,18 @@ __attribute__((amdgpu_waves_per_eu(G > 1 ? 1 : Cfg::WAVES))) void sched_kernel(S
     }
   if (xb) atomicOr(&s_bits[0], xb);
   if (yb) atomicOr(&s_bits[1], yb);
-  if (__any(chg_bits) && lane == 0) {
-    atomicOr(a.rowchg + tr, 1);
-    atomicOr(a.colchg + tc, 1);
-  }
-  if (__any(chg_test) && lane == 0) atomicOr(a.conv, 1);
+  if (__any(chg_bits) && lane == 0) s_chg[0] = 1;
+  if (__any(chg_test) && lane == 0) s_chg[1] = 1;
   __syncthreads();
+  // one atomic per tile and flag: the memory takes those to one address at 3 ns
+  // each
+  if (tid_all == 0) {
+    if (s_chg[0]) {
+      atomicOr(a.rowchg + tr, 1);
+      atomicOr(a.colchg + tc, 1);
+    }
+    if (s_chg[1]) atomicOr(a.conv, 1);
+  }
   const int sx = col0 / 16 + tid, sy = row0 / 16 + (tid - XS);
   if (active && tid < XS) {
     if (sx < a.slabs) a.xocc_out[(int64_t)tr * a.slabs + sx] = (s_bits[0] >> tid) & 1u;
@@ -228,19 +237,32 @@ constexpr int SP_B = 8;                // changed entries per thread per batch
 
 // (tile, slab) pairs the tiled kernel would compute in this squaring: dirty
 // tiles times the slabs occupied on both sides, plus two per dirty tile for
-// its epilogue.  One wave per tile, its lanes over the slabs.
+// its epilogue.  One wave per tile, its lanes over the slabs; one atomic per
+// workgroup (all go to one address, where the memory takes one every 3 ns: one
+// per wave made this 48 us at n = 4096).
 __global__ __launch_bounds__(EW) void tiled_work_kernel(SchedArgs a) {
+  __shared__ int s_wave[EW / 64];
   if (a.conv_prev && *a.conv_prev == 0) return;
-  const int t = bid_x() * (EW / 64) + tid_x() / 64, lane = tid_x() % 64;
-  if (t >= a.tiles_r * a.tiles_c) return;  // whole waves leave
-  const int tr = t / a.tiles_c, tc = t % a.tiles_c;
-  if (a.rowchg_prev && !a.rowchg_prev[tr] && !a.colchg_prev[tc]) return;  // clean tile
-  const uint8_t *xo = a.xocc_in + (int64_t)tr * a.slabs;
-  const uint8_t *yo = a.yocc_in + (int64_t)tc * a.slabs;
+  const int wave = tid_x() / 64, lane = tid_x() % 64;
+  const int t = bid_x() * (EW / 64) + wave;
   int cnt = 0;
-  for (int s = lane; s < a.slabs; s += 64) cnt += xo[s] & yo[s];
-  for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
-  if (lane == 0) atomicAdd(a.work, (unsigned long long)(cnt + 2));
+  if (t < a.tiles_r * a.tiles_c) {
+    const int tr = t / a.tiles_c, tc = t % a.tiles_c;
+    if (!a.rowchg_prev || a.rowchg_prev[tr] || a.colchg_prev[tc]) {  // not a clean tile
+      const uint8_t *xo = a.xocc_in + (int64_t)tr * a.slabs;
+      const uint8_t *yo = a.yocc_in + (int64_t)tc * a.slabs;
+      for (int s = lane; s < a.slabs; s += 64) cnt += xo[s] & yo[s];
+      for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
+      cnt += 2;
+    }
+  }
+  if (lane == 0) s_wave[wave] = cnt;
+  __syncthreads();
+  if (tid_x() == 0) {
+    unsigned long long sum = 0;
+    for (int w = 0; w < EW / 64; ++w) sum += s_wave[w];
+    if (sum) atomicAdd(a.work, sum);
+  }
 }
 
 // Per row: entries other than the identity (rowptr[i], when the row-sparse

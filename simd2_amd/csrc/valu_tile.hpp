@@ -312,7 +312,7 @@ __device__ __forceinline__ void valu_tile(int R, int Cn, int K, const float *__r
 
 // Epilogue of a BM x BN tile from the thread's acc: (+) C, optional APLP
 // mapping, change test, store.  Every thread of the workgroup calls it
-// (the tile flag takes a barrier); only threads with `active` set store, tid
+// (the flags take a barrier); only threads with `active` set store, tid
 // being their index among the tile's threads.  *changed_slot (LDS) must be
 // cleared before a barrier that precedes this call.
 template <class Op, int BM, int BN, int TM, int TN, bool CHECKED, bool MASKED>
@@ -373,13 +373,15 @@ __device__ __forceinline__ void valu_epilogue(int R, int Cn, float *O, int64_t l
     }
 
   }
+  // One atomic per tile at most: the memory takes atomics to one address at
+  // 3 ns each, and one per wave held a 1024^2 squaring up by 10 us.
   if (e.flag || tile_flag) {
-    const bool any = __any(changed);
-    if (e.flag && any && (tid % warpSize) == 0) atomicMax(e.flag, e.step);
-    if (tile_flag) {
-      if (any && (tid % warpSize) == 0) atomicOr(changed_slot, 1);
-      __syncthreads();
-      if (active && tid == 0) *tile_flag = *changed_slot;
+    if (__any(changed) && (tid % warpSize) == 0) *changed_slot = 1;
+    __syncthreads();
+    if (active && tid == 0) {
+      const int any = *changed_slot;
+      if (e.flag && any) atomicMax(e.flag, e.step);
+      if (tile_flag) *tile_flag = any;
     }
   }
 }
