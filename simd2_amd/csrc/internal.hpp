@@ -194,7 +194,8 @@ struct SchedArgs {
   int *colchg;
   const int *conv_prev;         // change-test flag of the previous squaring (null: first)
   int *conv;                    // change-test flag (check mode) of this squaring
-  unsigned long long *stats;    // optional: [0] tiles computed, [1] slab-tiles computed,
+  unsigned long long *stats;    // optional: [0] tiles computed, [1] slab-tiles computed (a
+                                //   tile stored as its mirror too counts as two),
                                 //   [2] / [3] rows / entries of row-sparse squarings,
                                 //   [4] / [5] rows / entries of changed-entry squarings
   // Sparse squarings, one workgroup per row over a list of entries built
@@ -213,9 +214,12 @@ struct SchedArgs {
   // per listed entry, cost_changed_entry per changed entry, plus cost_list
   // for either sparse form.
   const float *prev;  // null: no changed-entry form for this squaring
-  const int *asym;    // 0: the input of the loop is symmetric (null: unknown)
+  const int *asym;    // 0: the input of the loop is symmetric (null: unknown):
+                      //   the tiled kernel then computes one tile of each
+                      //   mirrored pair, if the tiles are square
   int rows_limit, changed_limit;
   int rows_auto, changed_auto;
+  int square;         // the tile shape is square
   float cost_slab_tile, cost_row_entry, cost_changed_entry, cost_list;
   unsigned long long *work;
   int *sq_mode;

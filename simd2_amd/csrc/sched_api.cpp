@@ -173,13 +173,17 @@ int simd2_converge_scheduled(int op, int n, float *X, int ldx, int do_epilogue,
   fills.add(conv, max_itr + 1, 0);
   fills.add(work, 2 * (int64_t)(max_itr + 1), 0);
   fills.add(mode, max_itr + 1, 0);
-  fills.add(stats, 12, 0);  // 6 64-bit counters
+  // asym and, right behind it, the 6 64-bit counters
+  fills.add(asym, (int64_t)((L.stats - L.asym) / sizeof(int)) + 12, 0);
   hipError_t e = launch_fill_multi(fills, stream);
   if (e == hipSuccess) e = launch_permute_copy(buf[0], L.P, X, ldx, n, perm, 0, stream);
-  // a symmetric input stays symmetric (every (x) here commutes bit for bit),
-  // which the changed-entry form can use
-  if (e == hipSuccess && changed_on) e = launch_fill_i32(asym, 0, 1, stream);
-  if (e == hipSuccess && changed_on) e = launch_sched_symmetry(buf[0], L.P, n, asym, stream);
+  // A symmetric input stays symmetric (every (x) here commutes bit for bit),
+  // which the changed-entry form and, with square tiles, the tiled form can
+  // use; the latter gains once the tiles are more than the CUs (grid graphs,
+  // n = 1100: 717 -> 607 us; n = 2000 1535 -> 1330; n = 1024 has one per CU).
+  // The check takes 5 us, 37 at n = 4096.
+  const bool sym_on = changed_on || (ci.bm == ci.bn && L.tiles_r * L.tiles_c > device_cu_count());
+  if (e == hipSuccess && sym_on) e = launch_sched_symmetry(buf[0], L.P, n, asym, stream);
   if (e == hipSuccess)
     e = launch_sched_occupancy(op, cfg, buf[0], L.P, n, L.tiles_r, L.tiles_c, L.slabs, xocc[0],
                                yocc[0], nullptr, stream);
@@ -217,11 +221,12 @@ int simd2_converge_scheduled(int op, int n, float *X, int ldx, int do_epilogue,
       // the previous squaring's input is the buffer this one overwrites; it
       // is read (to list the changed entries) before anything is written
       a.prev = changed_on && s > 0 ? a.nxt : nullptr;
-      a.asym = changed_on ? asym : nullptr;
+      a.asym = sym_on ? asym : nullptr;
       a.rows_limit = rows_on ? per_row * n : 0;
       a.changed_limit = a.prev ? changed_per_row * n : 0;
       a.rows_auto = rows_auto ? 1 : 0;
       a.changed_auto = changed_auto ? 1 : 0;
+      a.square = ci.bm == ci.bn;
       a.cost_slab_tile = (float)(16.0 * ci.bm * ci.bn * ps_term);
       a.cost_list = (float)((double)n * n * PS_LIST_ELEM);
       a.cost_row_entry = (float)(n * PS_ROW_ENTRY_COL);

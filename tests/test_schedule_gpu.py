@@ -200,3 +200,34 @@ def test_two_group_split_matches_plain_loop(gpu, kind):
                                                tile_config=1)
         assert st2 == simd2_amd.SUCCESS and itr2 == itr, (itr2, itr)
         assert torch.equal(Z.view(torch.int32), Y.view(torch.int32))
+
+
+@pytest.mark.parametrize("op,epi,check", OPS)
+@pytest.mark.parametrize("cfg,n", [(1, 1090), (1, 1345), (1, 2101), (0, 2117)])
+def test_symmetric_matrices_take_half_the_tiles(gpu, op, epi, check, cfg, n):
+    """More square tiles than CUs: of a symmetric matrix one tile of each pair
+    is computed and stored as both (split in four, in two and whole 64x64 tiles,
+    128x128 ones, sizes off every grid), of one that is not every tile.  Blocks
+    of vertices without an edge keep slabs empty."""
+    torch = gpu
+    X = family(torch, "grid", op, n, n)
+    ident = float("inf") if op.startswith("min") else float("-inf")
+    X[300:420, :] = ident
+    X[:, 300:420] = ident
+    assert torch.equal(X, X.t())
+    for skew in (False, True):
+        if skew:  # one entry, in the last row and column
+            X[n - 1, n - 2] = 50.0
+        assert torch.equal(X, X.t()) != skew
+        # a graph with cycles has no longest paths: a few squarings of those
+        cap = 3 if op == "max_plus" else 64
+        Y, itr, st = plain(torch, op, X, epi, check, max_itr=cap)
+        for rs, cs in ((0, 0), (-1, -1)):
+            Z, itr2, st2, rep = converge_scheduled(op, X.clone(), epilogue=epi, check=check,
+                                                   max_itr=cap, tile_config=cfg, row_sparse=rs,
+                                                   changed_sparse=cs)
+            assert (itr2, st2) == (itr, st), (skew, rs)
+            assert torch.equal(Z, Y), (skew, rs)
+            if rs == 0:  # the report counts a mirrored tile as two
+                assert 0 < rep["tiles_computed"] <= rep["tiles_total"]
+                assert rep["slab_tiles_computed"] < rep["slab_tiles_total"]
