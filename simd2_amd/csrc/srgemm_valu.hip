@@ -57,7 +57,165 @@ __attribute__((amdgpu_waves_per_eu(WAVES))) void srgemm_valu_kernel(
                                                                row0, col0, flag, sm);
 }
 
-// Small problems (at most four 64x64 tiles per CU; n = 1024 has one): the K
+// The smallest problems (up to one 64x64 tile per CU) on whole tiles and slabs:
+// eight waves per 64x64 tile, each on its own range of slabs with 8x8 outputs
+// per lane and its own LDS, so that no barrier holds the waves together; their
+// partial tiles are combined in wave order, ((p0 (+) p1) (+) p2) ..., before
+// the epilogue.  Only where (+) is min or max, which is exact: regrouping the
+// terms changes no bit.  Bound: VALU issue at two waves per SIMD; four groups
+// of 256 threads with 4x4 outputs per lane (the split kernel below) read LDS
+// twice as often per term and meet at 1024-thread barriers: 1024^3 41 us, here
+// 36.  With more tiles a second wave per SIMD hides less than those groups do,
+// and so do the masked loads off the grid (1000x1000x700 33 us, 36 this way).
+constexpr int WT = 64, WTM = 8, WBK = 16;
+constexpr int WG = 8;  // waves per tile
+
+struct WaveSmem {
+  __attribute__((aligned(16))) float Xs[2][WBK][WT + 4];
+  __attribute__((aligned(16))) float Ys[2][WBK][WT];
+};
+
+// acc = the slabs [kt0, kt1) of the tile at X's row and Y's column.  The LDS
+// slabs are the wave's own and its LDS instructions execute in order, so
+// nothing waits at a barrier: the fragments of a k pair are read while the pair
+// before it is computed, the next slab is written to the other buffer in the
+// middle of this one and the slab after it requested from memory.
+template <class Op>
+__device__ __forceinline__ void wave_loop(WaveSmem &sm, float (&acc)[WTM][WTM],
+                                          const float *__restrict__ X, int64_t ldx,
+                                          const float *__restrict__ Y, int64_t ldy, int kt0,
+                                          int kt1, int lane) {
+  const int tx = lane % 8, ty = lane / 8;
+#pragma unroll
+  for (int i = 0; i < WTM; ++i)
+#pragma unroll
+    for (int j = 0; j < WTM; ++j) acc[i][j] = Op::identity;
+  if (kt1 <= kt0) return;
+  vf4 xv[4], yv[4];
+  auto load = [&](int kt) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      xv[h] = *reinterpret_cast<const vf4u *>(X + (int64_t)(lane / 4 + 16 * h) * ldx + kt * WBK +
+                                              lane % 4 * 4);
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+      yv[h] = *reinterpret_cast<const vf4u *>(Y + (int64_t)(kt * WBK + lane / 16 + 4 * h) * ldy +
+                                              lane % 16 * 4);
+  };
+  auto store = [&](int buf) {
+    store_slab<WT, WT, WBK, 64, WT + 4>(sm.Xs[buf], sm.Ys[buf], xv, yv, lane);
+  };
+  float a[2][2][WTM], b[2][2][WTM];  // [set][k of the pair][...]
+  auto read = [&](int set, int buf, int kp) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        *reinterpret_cast<vf4 *>(&a[set][k][g * 4]) =
+            *reinterpret_cast<const vf4 *>(&sm.Xs[buf][2 * kp + k][g * 32 + ty * 4]);
+        *reinterpret_cast<vf4 *>(&b[set][k][g * 4]) =
+            *reinterpret_cast<const vf4 *>(&sm.Ys[buf][2 * kp + k][g * 32 + tx * 4]);
+      }
+  };
+  load(kt0);
+  store(0);
+  load(min(kt0 + 1, kt1 - 1));
+  read(0, 0, 0);
+  for (int kt = kt0; kt < kt1; ++kt) {
+    const int buf = (kt - kt0) & 1;
+#pragma unroll
+    for (int kp = 0; kp < WBK / 2; ++kp) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (kp == WBK / 4) {
+        store(buf ^ 1);
+        load(min(kt + 2, kt1 - 1));
+      }
+      const int s = kp & 1;
+      if (kp + 1 < WBK / 2) read(s ^ 1, buf, kp + 1);
+      else read(s ^ 1, buf ^ 1, 0);
+#pragma unroll
+      for (int i = 0; i < WTM; ++i)
+#pragma unroll
+        for (int j = 0; j < WTM; ++j) {
+          if constexpr (is_fused<Op>::value)
+            acc[i][j] = Op::fma_step(Op::fma_step(acc[i][j], a[s][0][i], b[s][0][j]), a[s][1][i],
+                                     b[s][1][j]);
+          else
+            acc[i][j] = Op::add3(acc[i][j], Op::mul(a[s][0][i], b[s][0][j]),
+                                 Op::mul(a[s][1][i], b[s][1][j]));
+        }
+    }
+  }
+}
+
+template <class Op>
+__global__ __launch_bounds__(64 * WG) __attribute__((amdgpu_waves_per_eu(2))) void
+srgemm_wave_kernel(int K, const float *__restrict__ X, int64_t ldx, const float *__restrict__ Y,
+                   int64_t ldy, float *O, int64_t ldo, Epilogue e, int tiles_r, int tiles_c) {
+  __shared__ WaveSmem sm[WG];
+  __shared__ int any_changed;
+  if (flag_done(e.flag, e.step)) return;
+  int tr, tc;
+  map_tile(bid_x(), tiles_r, tiles_c, tr, tc);
+  const int row0 = tr * WT, col0 = tc * WT;
+  const int lane = tid_x() % 64, w = __builtin_amdgcn_readfirstlane(tid_x() / 64);
+  const int slabs = K / WBK, per = (slabs + WG - 1) / WG;
+  const int kt0 = min(w * per, slabs), kt1 = min(kt0 + per, slabs);
+  if (tid_x() == 0) any_changed = 0;
+  float acc[WTM][WTM];
+  wave_loop<Op>(sm[w], acc, X + (int64_t)row0 * ldx, ldx, Y + col0, ldy, kt0, kt1, lane);
+  // every wave parks its partial tile in its own slabs and finishes one of the
+  // register tile's rows
+  static_assert(WTM * WTM * 64 * sizeof(float) <= sizeof(WaveSmem), "partial tile");
+  static_assert(WTM == WG, "one row of the register tile per wave");
+  vf4 *part = reinterpret_cast<vf4 *>(&sm[w]);
+#pragma unroll
+  for (int i = 0; i < WTM; ++i)
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+      part[(i * 2 + g) * 64 + lane] =
+          vf4{acc[i][g * 4], acc[i][g * 4 + 1], acc[i][g * 4 + 2], acc[i][g * 4 + 3]};
+  // C and the previous values travel while the partial tiles are combined (a
+  // squaring loop passes the same matrix as both)
+  const int tx = lane % 8, ty = lane / 8;
+  const int r = row0 + w / 4 * 32 + ty * 4 + w % 4;
+  vf4 cv[2], pv[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const int c = col0 + g * 32 + tx * 4;
+    cv[g] = pv[g] = vf4{0.f, 0.f, 0.f, 0.f};
+    if (e.C) cv[g] = *reinterpret_cast<const vf4u *>(e.C + (int64_t)r * e.ldc + c);
+    if (e.P == e.C && e.ldp == e.ldc) pv[g] = cv[g];
+    else if (e.P) pv[g] = *reinterpret_cast<const vf4u *>(e.P + (int64_t)r * e.ldp + c);
+  }
+  __syncthreads();
+  bool changed = false;
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < WG; ++q) {
+      const vf4 p = reinterpret_cast<const vf4 *>(&sm[q])[(w * 2 + g) * 64 + lane];
+#pragma unroll
+      for (int z = 0; z < 4; ++z) v[z] = q == 0 ? p[z] : Op::add(v[z], p[z]);
+    }
+#pragma unroll
+    for (int z = 0; z < 4; ++z) {
+      if (e.C) v[z] = Op::add(v[z], cv[g][z]);
+      if (e.mode == CHECK_APLP && v[z] > -1.0f && v[z] < 1.0f) v[z] = -FLT_MAX;
+      if (e.P) changed |= differs(v[z], pv[g][z], e.mode);
+    }
+    *reinterpret_cast<vf4u *>(O + (int64_t)r * ldo + col0 + g * 32 + tx * 4) =
+        vf4u{v[0], v[1], v[2], v[3]};
+  }
+  if (e.flag) {  // one atomic per tile at most (valu_epilogue)
+    if (__any(changed) && lane == 0) any_changed = 1;
+    __syncthreads();
+    if (tid_x() == 0 && any_changed) atomicMax(e.flag, e.step);
+  }
+}
+
+// Small problems (at most four 64x64 tiles per CU): the K
 // loop of each tile is split over G groups of 256 threads in one workgroup
 // (G = 4 up to two tiles per CU, else 2), each over a contiguous range of
 // slabs with its own LDS buffers, and the partial tiles are combined in
@@ -116,7 +274,7 @@ __global__ __launch_bounds__(256 * SK_GROUPS) void srgemm_valu_splitk_kernel(
                                                                g == 0);
 }
 
-// groups 4 or 2: whole tiles and slab groups; -4 or -2: the
+// groups 8: the wave kernel; 4 or 2: whole tiles and slab groups; -4 or -2: the
 // ragged form of as many groups.
 template <class Op>
 hipError_t launch_splitk(int R, int Cn, int K, const float *X, int64_t ldx, const float *Y,
@@ -124,7 +282,10 @@ hipError_t launch_splitk(int R, int Cn, int K, const float *X, int64_t ldx, cons
                          hipStream_t s) {
   const int tiles_r = (R + CfgS::BM - 1) / CfgS::BM, tiles_c = (Cn + CfgS::BN - 1) / CfgS::BN;
   const dim3 grid(tiles_r * tiles_c);
-  if (groups == 4)
+  if (groups == WG)
+    srgemm_wave_kernel<Op><<<grid, dim3(64 * WG), 0, s>>>(K, X, ldx, Y, ldy, O, ldo, e, tiles_r,
+                                                          tiles_c);
+  else if (groups == 4)
     srgemm_valu_splitk_kernel<Op, 4, false><<<grid, dim3(1024), 0, s>>>(
         R, Cn, K, X, ldx, Y, ldy, O, ldo, e, tiles_r, tiles_c);
   else if (groups == 2)
@@ -230,13 +391,19 @@ int valu_pick_cfg(int op, int R, int Cn, int K) {
 }
 
 // How a min / max semiring splits K where the 64x64 tiles were chosen and are
-// few: 4 / 2 groups of 256 threads, up to two / four tiles per CU, negative off
-// the grid (1025x1023x1021 77 us; 1999x1801x777 104, 111 unsplit); 0 -- unsplit.
+// few: 8 -- the wave kernel, on whole tiles and slabs up to one tile per CU with
+// at least two slabs a wave (64x64x1024 36.8 us in four groups, 31.7; 512^3 21.5
+// and 19.6; 1024x1024x256 15.0 and 14.0; x128 9.8 both); 4 / 2 -- groups of
+// 256 threads, up to two / four tiles per CU, negative off the grid
+// (1025x1023x1021 77 us; 1999x1801x777 104, 111 unsplit); 0 -- unsplit.
 static int splitk_groups(int op, int R, int Cn, int K, const Epilogue &e) {
   if (op == 1 || op == 8 || op < 0 || op > 6 || e.gate || K <= 0) return 0;
   const int64_t tiles =
       (int64_t)((R + CfgS::BM - 1) / CfgS::BM) * ((Cn + CfgS::BN - 1) / CfgS::BN);
   const int64_t cus = device_cu_count();
+  if (R % WT == 0 && Cn % WT == 0 && K % WBK == 0 && K >= 2 * WBK * WG && tiles <= cus &&
+      !e.tile_flags)
+    return WG;
   const int groups = tiles < 2 * cus ? 4 : tiles <= 4 * cus ? 2 : 0;
   if (groups == 0) return 0;
   if (R % CfgS::BM == 0 && Cn % CfgS::BN == 0 && K % (CfgS::BK * groups) == 0) return groups;

@@ -1,6 +1,7 @@
-"""The VALU product on rows of any alignment, in every form (split K in four
-and two groups, unsplit tiles), bit for bit against the oracle (minus_square on
-integers, which are exact)."""
+"""The small forms of the VALU product, bit for bit against the oracle
+(minus_square on integers, which are exact): the eight-wave K split (whole tiles
+and slabs, K >= 256, at most one 64x64 tile per CU) at the ends of its ranges and
+just off them, and rows of any alignment in every form."""
 import numpy as np
 import pytest
 import torch
@@ -9,6 +10,8 @@ import oracle
 import simd2_amd
 
 pytestmark = pytest.mark.gpu
+
+OPS = ["min_plus", "max_plus", "max_min", "max_mul", "min_mul", "min_max"]
 
 
 def _inputs(op, m, n, k, seed):
@@ -42,6 +45,18 @@ def _run(op, A, B, C, epi, pads, shift):
     return d[:, :n].cpu().numpy()
 
 
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("m,n,k", [(64, 64, 256), (64, 64, 240), (128, 64, 272), (64, 128, 271),
+                                   (65, 64, 256), (64, 63, 640), (128, 192, 1040),
+                                   (1024, 1024, 512)])
+def test_eight_waves(op, m, n, k):
+    A, B, C = _inputs(op, m, n, k, m + n + k)
+    for epi in (False, True):
+        want = oracle.srgemm_f32(op, A, B, C, epi)
+        assert np.array_equal(_run(op, A, B, C, epi, (0, 0, 0), 0), want)
+        assert np.array_equal(_run(op, A, B, C, epi, (3, 1, 5), 1), want)
+
+
 @pytest.mark.parametrize("op", ["min_plus", "max_mul", "minus_square"])
 @pytest.mark.parametrize("m,n,k", [(64, 64, 64), (70, 61, 33), (100, 129, 17), (1100, 1090, 40),
                                    (1500, 1600, 21), (2500, 2400, 18)])
@@ -53,3 +68,16 @@ def test_unaligned_rows(op, m, n, k):
         rows = np.unique(np.linspace(0, m - 1, 40).astype(int))
         assert np.array_equal(D[rows], oracle.srgemm_f32(op, A[rows], B, C[rows], True))
 
+
+@pytest.mark.parametrize("n", [512, 515, 1024])
+def test_loop_uses_the_change_test(n):
+    """The fused loop's flag comes from the eight-wave kernel's epilogue."""
+    rng = np.random.default_rng(n)
+    X = np.full((n, n), np.inf, np.float32)
+    mask = rng.random((n, n)) < 0.02
+    X[mask] = rng.integers(1, 101, int(mask.sum()))
+    np.fill_diagonal(X, 0)
+    Y, itr, st = simd2_amd.converge("min_plus", torch.from_numpy(X).cuda(), check="threshold")
+    Z, itr_r, st_r = simd2_amd.converge("min_plus", torch.from_numpy(X).cuda(),
+                                        check="threshold", flags=simd2_amd.CONVERGE_REFERENCE)
+    assert (st, itr) == (0, itr_r) and st_r == 0 and torch.equal(Y, Z)
