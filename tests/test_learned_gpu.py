@@ -139,3 +139,34 @@ def test_trained_network_replaces_flag_reads(gpu):
         covered += int(pred >= itr)
     assert covered >= 0.8 * len(specs), covered
     assert learned_reads <= 0.4 * plain_reads, (learned_reads, plain_reads)
+
+
+@pytest.mark.parametrize("n,kind", [(1025, "grid"), (1300, "path"), (1100, "hub 64"),
+                                    (1100, "hub 65"), (1100, "degree 29"), (1100, "degree 31"),
+                                    (2100, "parts"), (4096, "grid"), (4097, "grid")])
+def test_sparse_searches_match_oracle(gpu, oracle_learned, n, kind):
+    """n in (1024, 4096]: edge lists in LDS up to 30 (at 4096: 14) edges per vertex
+    on average and 64 per vertex, adjacency rows beyond; directed edges."""
+    torch = gpu
+    if kind == "grid":
+        X = grid_family(torch, "min_plus", n, 3)
+    else:
+        X = torch.full((n, n), float("inf"))
+        i = torch.arange(n - 1)
+        X[i, i + 1] = 1.0
+        if kind.startswith("hub"):
+            X[700, 10:10 + int(kind.split()[1])] = 2.0
+            X[700, 701] = float("inf")
+        elif kind.startswith("degree"):
+            for step in range(2, int(kind.split()[1]) + 1):
+                j = torch.arange(n)
+                X[j, (j + 31 * step) % n] = 3.0
+        elif kind == "parts":
+            X[:, 900:1400] = float("inf")
+            X[n - 1, 0] = 1.0
+        X.fill_diagonal_(0.0)
+        X = X.cuda()
+    print("searches", n, kind, flush=True)
+    f = LG.graph_features("min_plus", X, True).cpu().numpy()
+    fo = oracle_learned.graph_features("min_plus", X.cpu().numpy(), True)
+    np.testing.assert_allclose(f, fo, rtol=2e-6, atol=1e-7)
