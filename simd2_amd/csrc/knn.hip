@@ -56,6 +56,8 @@
 #include <hip/hip_bf16.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "internal.hpp"
 
 namespace simd2 {
@@ -514,7 +516,9 @@ __device__ __forceinline__ float fkey_inv(uint32_t k) {
 // thr[q] = (the ck-th smallest of the query's tile minima) + 2 E_q, +inf when
 // it has fewer than ck tiles; by bisection over the keys, one wave per query.
 // Also clears the query's candidate count and exact flag (and, in the first
-// wave, the counts of the overflow list and of the re-rank's LDS list).
+// wave, the counts of the overflow list and of the re-rank's LDS list).  Bound:
+// the ballots of the 32 bisection steps; with only the registers that hold keys
+// and no bounds in them 16384 queries of 256 tiles 35 -> 19 us.
 __global__ __launch_bounds__(256) void knn_tau_kernel(const float *__restrict__ tmin, int ntiles,
                                                       int Q, int ck, float e_coef,
                                                       const float *__restrict__ qn,
@@ -539,24 +543,31 @@ __global__ __launch_bounds__(256) void knn_tau_kernel(const float *__restrict__ 
   }
   float res = __builtin_inff();
   if (ntiles >= ck) {
-    while (lo < hi) {
-      const uint32_t mid = lo + (hi - lo) / 2;
-      int c = 0;
+    // keys past ntiles are above every mid; `held`: the registers that count
+    auto bisect = [&](auto held) {
+      while (lo < hi) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        int c = 0;
 #pragma unroll
-      for (int i = 0; i < TP; ++i)
-        c += (int)__popcll(__ballot(lane + 64 * i < ntiles && kv[i] <= mid));
-      if (ntiles > 64 * TP) {
-        int e = 0;
-        for (int j = lane + 64 * TP; j < ntiles; j += 64) e += fkey(t[j]) <= mid ? 1 : 0;
+        for (int i = 0; i < decltype(held)::value; ++i)
+          c += (int)__popcll(__ballot(kv[i] <= mid));
+        if (ntiles > 64 * TP) {
+          int e = 0;
+          for (int j = lane + 64 * TP; j < ntiles; j += 64) e += fkey(t[j]) <= mid ? 1 : 0;
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
-        c += e;
+          for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
+          c += e;
+        }
+        if (c >= ck)
+          hi = mid;
+        else
+          lo = mid + 1;
       }
-      if (c >= ck)
-        hi = mid;
-      else
-        lo = mid + 1;
-    }
+    };
+    if (ntiles <= 64 * TP / 2)
+      bisect(std::integral_constant<int, TP / 2>{});
+    else
+      bisect(std::integral_constant<int, TP>{});
     const float eq = e_coef * (qn[q] + *rnmax);
     res = fkey_inv(lo) + 2.0f * eq;
     res = res + fabsf(res) * 1e-6f;  // the sums above round by less than this
@@ -570,9 +581,9 @@ __global__ __launch_bounds__(256) void knn_tau_kernel(const float *__restrict__ 
 
 // --- canonical exact distances ---------------------------------------------------
 // The exact FP32 squared distance: eight partial sums s_p over dims j = p mod 8
-// in increasing j, combined as ((s0+s1)+(s2+s3))+((s4+s5)+(s6+s7)).  The wave
-// form (8 lanes per candidate, combined by xor shuffles 1, 2, 4) and this
-// thread form give the same bits.
+// in increasing j, combined as ((s0+s1)+(s2+s3))+((s4+s5)+(s6+s7)).  The form
+// of two lanes per candidate (exact_d32_pair) and this thread form give the
+// same bits.
 __device__ __forceinline__ float exact_d32_thread(const float *__restrict__ q,
                                                   const float *__restrict__ r, int d) {
   float s[8];
@@ -664,24 +675,46 @@ __device__ __forceinline__ double shfl_d(double v, int src) {
   return __longlong_as_double(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
 
-// Exact FP32 distances of candidates m0 .. m0 + 7 (lanes 8g .. 8g+7 sum dims
-// p, p + 8, ... of candidate m0 + g), combined by the xor tree; lane
-// 8g + p receives candidate m0 + g's distance.
-__device__ __forceinline__ float exact_d32_wave(const float *__restrict__ qrow,
-                                                const float *__restrict__ Rf, int64_t ldr, int d,
-                                                int r, bool live, int part) {
-  float s = 0.f;
+// The exact FP32 distance to `rrow` by two lanes: lane `half` sums the partial
+// sums s_p with p = 4 half .. 4 half + 3, 16 bytes of both rows at a time, and
+// both lanes get the result.  Bound: the candidates' rows, scattered over the
+// references and read through the L2; 32 candidates a wave keep 16 KiB of them
+// in flight at 128 dims (eight lanes per candidate and one word a load: 8
+// candidates, 100 us for 16384 queries of 128 dims, here 55).
+typedef float vf4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float exact_d32_pair(const float *__restrict__ qrow,
+                                                const float *__restrict__ rrow, int d, bool live,
+                                                int half) {
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
   if (live) {
-    const float *rrow = Rf + (int64_t)r * ldr;
-    for (int j = part; j < d; j += 8) {
-      const float t = qrow[j] - rrow[j];
-      s = s + t * t;
+    constexpr int U = 4;  // 8-dim groups loaded together
+    const float *q = qrow + 4 * half, *r = rrow + 4 * half;
+    int j = 0;
+    for (; j + 8 * U <= d; j += 8 * U) {
+      vf4u x[U], y[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        x[u] = *reinterpret_cast<const vf4u *>(q + j + 8 * u);
+        y[u] = *reinterpret_cast<const vf4u *>(r + j + 8 * u);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const float t = x[u][p] - y[u][p];
+          s[p] = s[p] + t * t;
+        }
     }
+    for (; j < d; j += 8)
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+        if (j + 4 * half + p < d) {
+          const float t = q[j + p] - r[j + p];
+          s[p] = s[p] + t * t;
+        }
   }
-  s += __shfl_xor(s, 1);
-  s += __shfl_xor(s, 2);
-  s += __shfl_xor(s, 4);
-  return s;
+  const float h = (s[0] + s[1]) + (s[2] + s[3]);
+  return h + __shfl_xor(h, 1);
 }
 
 // FP64 squared distance of reference r, summed by the whole wave.
@@ -721,12 +754,12 @@ __global__ __launch_bounds__(256) void rerank_small_kernel(
   if (exact) {
     if (lane < c) my_d = cand_d[(int64_t)q * CAND_CAP + lane];
   } else {
-    const int grp = lane / 8, part = lane % 8;
-    for (int m0 = 0; m0 < c; m0 += 8) {
-      const int r = __shfl(my_i, min(m0 + grp, 63));
-      const float s = exact_d32_wave(qrow, Rf, ldr, d, r, m0 + grp < c, part);
-      const float got = __shfl(s, 8 * ((lane - m0) & 7));
-      if (lane >= m0 && lane < m0 + 8 && lane < c) my_d = got;
+    for (int m0 = 0; m0 < c; m0 += 32) {
+      const int m = m0 + lane / 2;
+      const int r = __shfl(my_i, m);
+      const float s = exact_d32_pair(qrow, Rf + (int64_t)r * ldr, d, m < c, lane % 2);
+      const float got = __shfl(s, 2 * (lane & 31));
+      if (lane >= m0 && lane < m0 + 32 && lane < c) my_d = got;
     }
   }
   // bitonic sort of the wave by (distance, index); padding sorts last
@@ -824,30 +857,18 @@ __global__ __launch_bounds__(64) void rerank_big_kernel(const float *__restrict_
   const float *cd = cand_d + (int64_t)q * CAND_CAP;
   const int *ci = cand_i + (int64_t)q * CAND_CAP;
 
-  // Exact FP32 distances: lanes 8g .. 8g+7 sum dims p, p + 8, ... of
-  // candidate m0 + g (8 candidates in flight), combined by the xor tree.
+  // Exact FP32 distances, 32 candidates in flight.
   if (exact) {
     for (int m = lane; m < c; m += 64) {
       sd[m] = cd[m];
       si[m] = ci[m];
     }
   } else {
-    const int grp = lane / 8, part = lane % 8;
-    for (int m0 = 0; m0 < c; m0 += 8) {
-      const int m = m0 + grp;
+    for (int m0 = 0; m0 < c; m0 += 32) {
+      const int m = m0 + lane / 2;
       const int r = m < c ? ci[m] : 0;
-      float s = 0.f;
-      if (m < c) {
-        const float *rrow = Rf + (int64_t)r * ldr;
-        for (int j = part; j < d; j += 8) {
-          const float t = qrow[j] - rrow[j];
-          s = s + t * t;
-        }
-      }
-      s += __shfl_xor(s, 1);
-      s += __shfl_xor(s, 2);
-      s += __shfl_xor(s, 4);
-      if (part == 0 && m < c) {
+      const float s = exact_d32_pair(qrow, Rf + (int64_t)r * ldr, d, m < c, lane % 2);
+      if (lane % 2 == 0 && m < c) {
         sd[m] = s;
         si[m] = r;
       }

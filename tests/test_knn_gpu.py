@@ -304,3 +304,28 @@ def test_f2h_h2f_roundtrip(gpu):
     h = simd2_amd.f2h(x)
     assert gpu.equal(h, x.half())
     assert gpu.equal(simd2_amd.h2f(h), x.half().float())
+
+
+@pytest.mark.parametrize("d", [1, 5, 8, 13, 31, 32, 36, 63, 100, 128])
+def test_knn_bf16_reported_distances_are_the_canonical_sums(gpu, d):
+    """Dims off and on the 8-dim groups and their blocks of four, rows at any
+    word: the reported squared distances are the canonical FP32 sum's bits or,
+    for near ties, the FP64 distance rounded."""
+    from simd2_amd.knn import knn_bf16
+    torch = gpu
+    rng = np.random.default_rng(d)
+    R, Q, k = 700, 45, 9
+    data = rng.normal(size=(R + Q, d)).astype(np.float32)
+    wide = torch.zeros((R + Q) * (d + 3) + 1, device="cuda")[1:].view(R + Q, d + 3)
+    wide[:, :d] = torch.from_numpy(data).cuda()
+    dist, idx, _ = knn_bf16(wide[R:, :d], wide[:R, :d], k, sqrt=False)
+    dist, idx = dist.cpu().numpy(), idx.cpu().numpy().astype(np.int64)
+    diff = data[R:, None, :] - data[:R][idx]
+    s = np.zeros((8,) + idx.shape, np.float32)
+    for j in range(d):
+        s[j % 8] = s[j % 8] + diff[..., j] * diff[..., j]
+    want = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]))
+    d64 = ((data[R:, None, :].astype(np.float64) - data[:R][idx]) ** 2).sum(-1)
+    assert bool(((dist == want) | (dist == d64.astype(np.float32))).all())
+    full = ((data[R:, None, :].astype(np.float64) - data[None, :R]) ** 2).sum(-1)
+    assert np.array_equal(idx, np.argsort(full, axis=1, kind="stable")[:, :k])
