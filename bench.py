@@ -499,7 +499,7 @@ def batched_graphs(torch, simd2_amd, count=4096, seed=0, ceiling=None):
     cfg, launches = b.schedule()
     outs = [b.download(g) for g in range(count)]
 
-    # the per-graph loop (fused change test, one flag read per squaring)
+    # the per-graph loop (fused change test, squarings enqueued ahead of the flag read)
     work = {}
     flag = torch.zeros(1, dtype=torch.int32, device="cuda")
     singles, same_itr = [], 0
