@@ -395,7 +395,9 @@ int valu_pick_cfg(int op, int R, int Cn, int K) {
 // at least two slabs a wave (64x64x1024 36.8 us in four groups, 31.7; 512^3 21.5
 // and 19.6; 1024x1024x256 15.0 and 14.0; x128 9.8 both); 4 / 2 -- groups of
 // 256 threads, up to two / four tiles per CU, negative off the grid
-// (1025x1023x1021 77 us; 1999x1801x777 104, 111 unsplit); 0 -- unsplit.
+// (1025x1023x1021 77 us; 1999x1801x777 104, 111 unsplit), and no more than slabs
+// (16x16x16 7.4 us in four groups, 5.3 unsplit; 16x16x32 8.0, 5.8 in two, 6.2
+// unsplit; 1500x1400x32 9.8 in two, 9.1 unsplit); 0 -- unsplit.
 static int splitk_groups(int op, int R, int Cn, int K, const Epilogue &e) {
   if (op == 1 || op == 8 || op < 0 || op > 6 || e.gate || K <= 0) return 0;
   const int64_t tiles =
@@ -404,7 +406,8 @@ static int splitk_groups(int op, int R, int Cn, int K, const Epilogue &e) {
   if (R % WT == 0 && Cn % WT == 0 && K % WBK == 0 && K >= 2 * WBK * WG && tiles <= cus &&
       !e.tile_flags)
     return WG;
-  const int groups = tiles < 2 * cus ? 4 : tiles <= 4 * cus ? 2 : 0;
+  int groups = tiles < 2 * cus ? 4 : tiles <= 4 * cus ? 2 : 0;
+  if (K <= 2 * CfgS::BK) groups = K <= CfgS::BK || groups == 2 ? 0 : 2;
   if (groups == 0) return 0;
   if (R % CfgS::BM == 0 && Cn % CfgS::BN == 0 && K % (CfgS::BK * groups) == 0) return groups;
   return -groups;

@@ -57,6 +57,17 @@ def test_eight_waves(op, m, n, k):
         assert np.array_equal(_run(op, A, B, C, epi, (3, 1, 5), 1), want)
 
 
+@pytest.mark.parametrize("op", OPS)
+@pytest.mark.parametrize("m,n,k", [(16, 16, 16), (1, 1, 1), (65, 63, 10), (64, 64, 17), (100, 90, 32),
+                                   (64, 128, 33), (1500, 1400, 16), (1500, 1400, 32)])
+def test_no_more_groups_than_slabs(op, m, n, k):
+    A, B, C = _inputs(op, m, n, k, m + n + k)
+    rows = np.unique(np.linspace(0, m - 1, 40).astype(int))
+    for epi in (False, True):
+        D = _run(op, A, B, C, epi, (1, 0, 2), 1)
+        assert np.array_equal(D[rows], oracle.srgemm_f32(op, A[rows], B, C[rows], epi))
+
+
 @pytest.mark.parametrize("op", ["min_plus", "max_mul", "minus_square"])
 @pytest.mark.parametrize("m,n,k", [(64, 64, 64), (70, 61, 33), (100, 129, 17), (1100, 1090, 40),
                                    (1500, 1600, 21), (2500, 2400, 18)])
