@@ -217,7 +217,7 @@ srgemm_wave_kernel(int K, const float *__restrict__ X, int64_t ldx, const float 
 
 // Small problems (at most four 64x64 tiles per CU): the K
 // loop of each tile is split over G groups of 256 threads in one workgroup
-// (G = 4 up to two tiles per CU, else 2), each over a contiguous range of
+// (G: splitk_groups), each over a contiguous range of
 // slabs with its own LDS buffers, and the partial tiles are combined in
 // group order, ((p0 (+) p1) (+) p2) (+) p3, before the usual epilogue: G
 // times the resident waves.  Only for the semirings whose (+) is min or max,
@@ -393,11 +393,14 @@ int valu_pick_cfg(int op, int R, int Cn, int K) {
 // How a min / max semiring splits K where the 64x64 tiles were chosen and are
 // few: 8 -- the wave kernel, on whole tiles and slabs up to one tile per CU with
 // at least two slabs a wave (64x64x1024 36.8 us in four groups, 31.7; 512^3 21.5
-// and 19.6; 1024x1024x256 15.0 and 14.0; x128 9.8 both); 4 / 2 -- groups of
-// 256 threads, up to two / four tiles per CU, negative off the grid
-// (1025x1023x1021 77 us; 1999x1801x777 104, 111 unsplit), and no more than slabs
+// and 19.6; 1024x1024x256 15.0 and 14.0; x128 9.8 both); 4 or 2 -- groups of
+// 256 threads, negative off the grid; 0 -- unsplit, from four tiles per CU up
+// (1999x1801x777 104 us in two, 111 unsplit).  Four groups pay where a CU has
+// one workgroup, or two of the form without bounds, and each group some slabs
+// (1408^3 87 us in four, 92 in two; 1025x1023x1021 77 and 69; 1100x1000x200 27
+// and 21.5; 1024x1024x96 11.0 and 8.5).  Never more groups than slabs
 // (16x16x16 7.4 us in four groups, 5.3 unsplit; 16x16x32 8.0, 5.8 in two, 6.2
-// unsplit; 1500x1400x32 9.8 in two, 9.1 unsplit); 0 -- unsplit.
+// unsplit; 1500x1400x32 9.8 in two, 9.1 unsplit).
 static int splitk_groups(int op, int R, int Cn, int K, const Epilogue &e) {
   if (op == 1 || op == 8 || op < 0 || op > 6 || e.gate || K <= 0) return 0;
   const int64_t tiles =
@@ -406,11 +409,11 @@ static int splitk_groups(int op, int R, int Cn, int K, const Epilogue &e) {
   if (R % WT == 0 && Cn % WT == 0 && K % WBK == 0 && K >= 2 * WBK * WG && tiles <= cus &&
       !e.tile_flags)
     return WG;
-  int groups = tiles < 2 * cus ? 4 : tiles <= 4 * cus ? 2 : 0;
-  if (K <= 2 * CfgS::BK) groups = K <= CfgS::BK || groups == 2 ? 0 : 2;
-  if (groups == 0) return 0;
-  if (R % CfgS::BM == 0 && Cn % CfgS::BN == 0 && K % (CfgS::BK * groups) == 0) return groups;
-  return -groups;
+  if (tiles > 4 * cus || K <= CfgS::BK || (K <= 2 * CfgS::BK && tiles >= 2 * cus)) return 0;
+  const bool whole = R % CfgS::BM == 0 && Cn % CfgS::BN == 0;
+  const bool whole4 = whole && K % (CfgS::BK * 4) == 0;
+  if (K > 8 * CfgS::BK && (tiles <= cus || (tiles < 2 * cus && whole4))) return whole4 ? 4 : -4;
+  return whole && K % (CfgS::BK * 2) == 0 ? 2 : -2;
 }
 
 hipError_t launch_valu_f32(int op, int R, int Cn, int K, const float *X,

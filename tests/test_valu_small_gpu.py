@@ -59,8 +59,9 @@ def test_eight_waves(op, m, n, k):
 
 @pytest.mark.parametrize("op", OPS)
 @pytest.mark.parametrize("m,n,k", [(16, 16, 16), (1, 1, 1), (65, 63, 10), (64, 64, 17), (100, 90, 32),
-                                   (64, 128, 33), (1500, 1400, 16), (1500, 1400, 32)])
-def test_no_more_groups_than_slabs(op, m, n, k):
+                                   (64, 128, 33), (1500, 1400, 16), (1500, 1400, 32), (64, 64, 128),
+                                   (130, 70, 129), (1088, 1024, 192), (1088, 1020, 200)])
+def test_groups_by_slabs_and_tiles(op, m, n, k):
     A, B, C = _inputs(op, m, n, k, m + n + k)
     rows = np.unique(np.linspace(0, m - 1, 40).astype(int))
     for epi in (False, True):
