@@ -714,13 +714,21 @@ __device__ __forceinline__ float exact_d32_pair(const float *__restrict__ qrow,
           s[p] = s[p] + t * t;
         }
     }
-    for (; j < d; j += 8)
+    for (; j + 8 <= d; j += 8) {
+      const vf4u x = *reinterpret_cast<const vf4u *>(q + j);
+      const vf4u y = *reinterpret_cast<const vf4u *>(r + j);
 #pragma unroll
-      for (int p = 0; p < 4; ++p)
-        if (j + 4 * half + p < d) {
-          const float t = q[j + p] - r[j + p];
-          s[p] = s[p] + t * t;
-        }
+      for (int p = 0; p < 4; ++p) {
+        const float t = x[p] - y[p];
+        s[p] = s[p] + t * t;
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      if (j + 4 * half + p < d) {
+        const float t = q[j + p] - r[j + p];
+        s[p] = s[p] + t * t;
+      }
   }
   const float h = (s[0] + s[1]) + (s[2] + s[3]);
   return h + __shfl_xor(h, 1);
