@@ -75,6 +75,14 @@ struct WaveSmem {
   __attribute__((aligned(16))) float Ys[2][WBK][WT];
 };
 
+// Between LDS stores and reads of what other lanes of the same wave stored (or
+// the reverse).  A wave's LDS instructions execute in order, so this costs no
+// instruction: it keeps the compiler from moving one across the other.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // acc = the slabs [kt0, kt1) of the tile at X's row and Y's column.  The LDS
 // slabs are the wave's own and its LDS instructions execute in order, so
 // nothing waits at a barrier: the fragments of a k pair are read while the pair
@@ -119,6 +127,7 @@ __device__ __forceinline__ void wave_loop(WaveSmem &sm, float (&acc)[WTM][WTM],
   };
   load(kt0);
   store(0);
+  wave_lds_fence();
   load(min(kt0 + 1, kt1 - 1));
   read(0, 0, 0);
   for (int kt = kt0; kt < kt1; ++kt) {
@@ -127,7 +136,9 @@ __device__ __forceinline__ void wave_loop(WaveSmem &sm, float (&acc)[WTM][WTM],
     for (int kp = 0; kp < WBK / 2; ++kp) {
       __builtin_amdgcn_sched_barrier(0);
       if (kp == WBK / 4) {
+        wave_lds_fence();
         store(buf ^ 1);
+        wave_lds_fence();
         load(min(kt + 2, kt1 - 1));
       }
       const int s = kp & 1;
@@ -168,6 +179,7 @@ srgemm_wave_kernel(int K, const float *__restrict__ X, int64_t ldx, const float 
   // register tile's rows
   static_assert(WTM * WTM * 64 * sizeof(float) <= sizeof(WaveSmem), "partial tile");
   static_assert(WTM == WG, "one row of the register tile per wave");
+  wave_lds_fence();
   vf4 *part = reinterpret_cast<vf4 *>(&sm[w]);
 #pragma unroll
   for (int i = 0; i < WTM; ++i)
