@@ -675,11 +675,15 @@ __global__ __launch_bounds__(EW) void symmetrize_kernel(SchedArgs a, int bm, int
   }
 }
 
-// *asym = 1 when some D[r][c] differs from D[c][r] in its bits.
+// *asym = 1 when some D[r][c] differs from D[c][r] in its bits.  A workgroup
+// leaves when another has shown it, all of its waves on one reading of *asym:
+// it may be written meanwhile.
 __global__ __launch_bounds__(EW) void symmetry_check_kernel(const float *D, int64_t ld, int n,
                                                             int *asym) {
   __shared__ float ta[SY][SY + 1], tb[SY][SY + 1];
-  if (*asym) return;  // another tile has shown it
+  int known = 0;
+  if (tid_x() == 0) known = __hip_atomic_load(asym, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__syncthreads_or(known)) return;
   const int T = (n + SY - 1) / SY;
   int I, J;
   tile_pair(bid_x(), T, I, J);
@@ -691,6 +695,8 @@ __global__ __launch_bounds__(EW) void symmetry_check_kernel(const float *D, int6
     const int rl = e / SY, cl = e % SY;
     diff |= __float_as_uint(ta[rl][cl]) != __float_as_uint(tb[cl][rl]);
   }
+  // a plain store of the one value it can get: as an atomic of the device's
+  // scope it made an asymmetric 4096^2 52 us instead of 15 (symmetric: 39)
   if (__syncthreads_or(diff) && tid_x() == 0) *asym = 1;
 }
 

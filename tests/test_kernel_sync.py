@@ -31,3 +31,12 @@ def test_lds_exchange_of_the_wave_kernel_is_fenced():
     # the partial tile is parked over slabs that other lanes have read
     kernel = _body("srgemm_valu.hip", "srgemm_wave_kernel")
     assert re.search(r"wave_loop<Op>\([^;]*;.*?wave_lds_fence\(\);.*?\bpart\[", kernel, re.S)
+
+
+def test_symmetry_check_leaves_as_one_workgroup():
+    """Other workgroups write *asym during the launch, so waves may read different
+    values: the decision to leave is taken by the workgroup, after a barrier."""
+    body = _body("sched.hip", "symmetry_check_kernel")
+    before = body[:body.index("return;")]
+    assert "__syncthreads" in before and "__hip_atomic_load(asym" in before
+    assert not re.search(r"\*asym\b(?! = 1;)", body)
