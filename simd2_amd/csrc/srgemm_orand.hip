@@ -49,6 +49,7 @@ __device__ __forceinline__ bool flag_done(const FlagStep &f) {
 }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -118,6 +119,7 @@ __global__ __launch_bounds__(WR * WC * 64) void orand_packed_kernel(
   // bit 2 rb + h: A rows 32 rb.. hold a 1 in 64-k half h; bit 16 + 2 cb + h:
   // the same for B columns 32 cb..
   __shared__ uint32_t some[3];
+  __shared__ uint64_t occ[NT / 64];
   if (flag_done(flag)) return;
   const int tid = tid_x();
   const int lane = tid % 64;
@@ -228,33 +230,54 @@ __global__ __launch_bounds__(WR * WC * 64) void orand_packed_kernel(
             __builtin_shufflevector(b[h][j][0], b[h][j][1], 0, 1, 2, 3, -1, -1, -1, -1), acc[i][j],
             4, 4, 0, 0, 0, 0);
   };
-  if (nslab > 0) {
+  // Slabs are taken one after the other until the tile's A rows hold no 1 in two
+  // of them (or in the first two).  What is left is looked over SCAN slabs at a
+  // time, a wave reading whole rows with a slab per lane, and only those with a 1
+  // in A are taken: a slab that is merely loaded and converted costs 0.7 us of the
+  // 1.0 us of one that is multiplied.  8192^3, every slab taken and here: no bit at
+  // all 187 -> 45 us, blocks of 64 on the diagonal 187 -> 55, density 1e-5 188 ->
+  // 102, 1e-4 204 -> 210, 0.5 266 -> 272 (4096^3 38.3 -> 39).  A loop of its own
+  // for the second part would leave the first as it was, but needs a second set
+  // of accumulator registers.
+  constexpr int SCAN = 60;  // leaves lanes for the slabs asked for past the last
+  int count = nslab;        // slabs to take, the s-th (s < 64 but for all) ...
+  int order = kw0 + lane * OA_KW;  // ... from word order[s % 64] + (s - s % 64) * OA_KW
+  int rest = nslab;                // the first slab not looked at
+  for (bool all = true; count > 0; all = false) {
     // At slab s: its fragments are in registers, the fragments of s + 1 are
     // read from LDS between the products, the words of s + 2 are converted
     // into LDS and those of s + 4 are on their way from memory.  The waves
     // that stage A do so before their products, the others after, so that one
     // half converts while the other keeps the matrix cores busy.  `some` is
     // read one slab ahead too and cleared one slab before it is collected.
-    auto slab = [&](int s) { return kw0 + min(s, nslab - 1) * OA_KW; };
+    // Words past the last slab are kw_end or more: read from inside the matrix
+    // (load), A's taken as zero (stage).
+    auto word_of = [&](int s) {
+      return __builtin_amdgcn_readlane(order, s & 63) + (s & ~63) * OA_KW;
+    };
     if (tid < 3) some[tid] = 0;
-    uwords pre0 = load(slab(0)), pre1 = load(slab(1));
+    int kwa = word_of(0), kwb = word_of(1);
+    uwords pre0 = load(kwa), pre1 = load(kwb);
     __syncthreads();
-    stage(pre0, kw0, 0, 0);
-    stage(pre1, kw0 + OA_KW, 1, 1);
-    pre0 = load(slab(2));
-    pre1 = load(slab(3));
+    stage(pre0, kwa, 0, 0);
+    stage(pre1, kwb, 1, 1);
+    kwa = word_of(2), kwb = word_of(3);
+    pre0 = load(kwa);
+    pre1 = load(kwb);
     __syncthreads();
     fragments(0, 0);
     fragments(0, 1);
-    uint32_t on = some[0];
+    uint32_t on = some[0], now = 0;
+    constexpr uint32_t a_bits = 0xffffu;
+    const bool none = !(__builtin_amdgcn_readfirstlane(on | some[1]) & a_bits);
     __syncthreads();
     int slot = 0;  // s % 3
-    auto step = [&](int s, uwords &pre) {
+    auto step = [&](int s, uwords &pre, int &kw) {
       const int buf = s & 1, s1 = slot == 2 ? 0 : slot + 1, s2 = s1 == 2 ? 0 : s1 + 1;
-      const uint32_t now = __builtin_amdgcn_readfirstlane(on);
+      now = __builtin_amdgcn_readfirstlane(on);
       on = some[s1];
       if (tid == 0) some[slot] = 0;
-      if (stage_a) stage(pre, kw0 + (s + 2) * OA_KW, buf, s2);
+      if (stage_a) stage(pre, kw, buf, s2);
       multiply(now, 0);
       __builtin_amdgcn_sched_barrier(0);
       fragments(buf ^ 1, 0);
@@ -262,14 +285,48 @@ __global__ __launch_bounds__(WR * WC * 64) void orand_packed_kernel(
       multiply(now, 1);
       __builtin_amdgcn_sched_barrier(0);
       fragments(buf ^ 1, 1);
-      if (!stage_a) stage(pre, kw0 + (s + 2) * OA_KW, buf, s2);
-      pre = load(slab(s + 4));
+      if (!stage_a) stage(pre, kw, buf, s2);
+      kw = word_of(s + 4);
+      pre = load(kw);
       slot = s1;
       __syncthreads();
     };
-    for (int s = 0; s < nslab; s += 2) {
-      step(s, pre0);
-      if (s + 1 < nslab) step(s + 1, pre1);
+    int s = all && none ? 2 : 0, end = s ? 0 : count;
+    while (s < end) {
+      step(s, pre0, kwa);
+      const uint32_t was = now;
+      if (s + 1 < count) step(s + 1, pre1, kwb);
+      s += 2;
+      end = all && !((was | now) & a_bits) ? 0 : end;
+    }
+    if (end == 0) rest = s;
+    for (count = 0; count == 0 && rest < nslab; rest += SCAN) {
+      constexpr int ROWS = BM * 64 / NT, BATCH = 8;
+      const int w = min(kw0 + (rest + lane) * OA_KW, nkw - OA_KW);  // nkw >= 4: nslab > 2
+      uint32_t any = 0;
+#pragma unroll 1
+      for (int i = 0; i < ROWS; i += BATCH) {
+        u32x4u v[BATCH];
+#pragma unroll
+        for (int q = 0; q < BATCH; ++q)
+          v[q] = *reinterpret_cast<const u32x4u *>(
+              A + (uint64_t)(uint32_t)min(row0 + wave * ROWS + i + q, M - 1) * lda + w);
+#pragma unroll
+        for (int q = 0; q < BATCH; ++q) any |= v[q][0] | v[q][1] | v[q][2] | v[q][3];
+      }
+      const uint64_t mine = __ballot(any != 0u && lane < SCAN && rest + lane < nslab);
+      if (lane == 0) occ[wave] = mine;
+      __syncthreads();
+      uint64_t full = 0;
+#pragma unroll
+      for (int q = 0; q < NT / 64; ++q) full |= occ[q];
+      __syncthreads();
+      // the slabs taken go to the first lanes in order, the others' lanes get kw_end
+      const int rank = __popcll(full & ((1ull << lane) - 1));
+      const bool taken = full >> lane & 1;
+      count = __builtin_amdgcn_readfirstlane(__popcll(full));
+      order = __builtin_amdgcn_ds_permute((taken ? rank : count + lane - rank) * 4,
+                                          taken ? kw0 + (rest + lane) * OA_KW : kw_end);
     }
   }
 
