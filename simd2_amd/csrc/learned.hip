@@ -98,9 +98,9 @@ __global__ __launch_bounds__(256) void in_degree_kernel(const float *X, int64_t 
 // adjacency: out[0] += edges (i, j), out[1] += those with (j, i) an edge too.
 // Thread t takes words t, t + 256, ... of row i and tests bit i of each
 // listed row j.
-__global__ __launch_bounds__(256) void symmetry_kernel(const uint32_t *__restrict__ adj, int n,
-                                                       int nw, int step, int *out) {
-  const int i = bid_x() * step;
+__device__ __forceinline__ void count_symmetry(int k, const uint32_t *__restrict__ adj, int n,
+                                               int nw, int step, int *out) {
+  const int i = k * step;
   if (i >= n) return;
   int e = 0, s = 0;
   for (int w = tid_x(); w < nw; w += 256) {
@@ -131,22 +131,23 @@ __global__ __launch_bounds__(256) void pack_adj_kernel(const float *X, int64_t l
 
 // Breadth-first search from src over the packed adjacency, by one
 // workgroup.  The frontier is a vertex list in global memory (cur / nxt, n
-// ints each); thread t owns adjacency words t + 256 q.  Writes depth (the
+// ints each); thread t of T owns adjacency words t + T q.  Writes depth (the
 // last level reached), reached (vertex count) and the lowest-numbered vertex
 // of the last level to res[0..2] and, when level is set, each vertex's level
 // (-1: unreached).  Every level adds at least one vertex or ends the search,
 // so it stops within n levels.  s_cnt: 3 ints of LDS.
+template <int T>
 __device__ void bfs(const uint32_t *adj, int n, int nw, int src, int *cur, int *nxt, int *level,
                     int *res, uint32_t *visited, uint32_t *red, int *s_cnt) {
   const int t = tid_x();
   // Short adjacency rows (nw <= 128 words, n <= 4096) would leave most
   // threads idle: the threads form G groups of wpg words, each group expands
   // its share of the frontier, and the groups' words are OR-ed through LDS.
-  const int wpg = nw <= 64 ? 64 : (nw <= 128 ? 128 : BFS_T);
-  const int G = BFS_T / wpg, g = t / wpg, tw = t % wpg;
-  for (int w = t; w < nw; w += BFS_T) visited[w] = 0;
+  const int wpg = nw <= 64 ? 64 : (nw <= 128 ? 128 : T);
+  const int G = T / wpg, g = t / wpg, tw = t % wpg;
+  for (int w = t; w < nw; w += T) visited[w] = 0;
   if (level)
-    for (int v = t; v < n; v += BFS_T) level[v] = v == src ? 0 : -1;
+    for (int v = t; v < n; v += T) level[v] = v == src ? 0 : -1;
   __syncthreads();
   if (t == 0) {
     visited[src / 32] |= 1u << (src % 32);
@@ -171,7 +172,7 @@ __device__ void bfs(const uint32_t *adj, int n, int nw, int src, int *cur, int *
       }
 #pragma unroll
       for (int q = 0; q < BFS_W; ++q) {
-        const int w = tw + BFS_T * q;
+        const int w = tw + T * q;
         if (w < nw) {
 #pragma unroll
           for (int k = 0; k < BFS_U; ++k)
@@ -179,7 +180,7 @@ __device__ void bfs(const uint32_t *adj, int n, int nw, int src, int *cur, int *
         }
       }
     }
-    if (G > 1) {  // nw <= wpg < BFS_T: one word per thread
+    if (G > 1) {  // nw <= wpg < T: one word per thread
       red[t] = acc[0];
       __syncthreads();
       if (g == 0)
@@ -187,7 +188,7 @@ __device__ void bfs(const uint32_t *adj, int n, int nw, int src, int *cur, int *
     }
 #pragma unroll
     for (int q = 0; q < BFS_W; ++q) {
-      const int w = tw + BFS_T * q;
+      const int w = tw + T * q;
       if (g == 0 && w < nw) {
         uint32_t fresh = acc[q] & ~visited[w];
         if (fresh) {
@@ -375,15 +376,14 @@ __host__ __device__ inline int sparse_cap(int n) {
   return fit < SL_E ? fit : SL_E;
 }
 
-// One wave per vertex: its out-neighbours to edge[], base << 13 | count to
-// row[], in any order of the vertices.  *total (0 beforehand) ends above cap
-// when the lists do not hold the graph; one atomic per workgroup.
-__global__ __launch_bounds__(256) void edge_list_kernel(const uint32_t *adj, int n, int nw, int cap,
-                                                        uint16_t *edge, uint32_t *row,
-                                                        int *total) {
+// One wave per vertex 4 k .. 4 k + 3: its out-neighbours to edge[], base << 13 |
+// count to row[], in any order of the vertices.  *total (0 beforehand) ends above
+// cap when the lists do not hold the graph; one atomic per workgroup.
+__device__ __forceinline__ void list_edges(int k, const uint32_t *adj, int n, int nw, int cap,
+                                           uint16_t *edge, uint32_t *row, int *total) {
   __shared__ int s_cnt[4], s_base;
   const int wave = tid_x() / 64, lane = tid_x() % 64;
-  const int v = bid_x() * 4 + wave;
+  const int v = k * 4 + wave;
   uint32_t m[SL_NW / 64];
   int mine = 0;
 #pragma unroll
@@ -419,6 +419,19 @@ __global__ __launch_bounds__(256) void edge_list_kernel(const uint32_t *adj, int
   if (lane == 0) row[v] = (uint32_t)base << 13 | (uint32_t)s_cnt[wave];
 }
 
+// What reads the finished adjacency, in one launch: the workgroups up to `rows`
+// count symmetry, the others list edges (a launch of its own for those cost
+// graphs too dense for the lists 5 to 13 us, half of that for the one that
+// then searched nothing).
+__global__ __launch_bounds__(256) void adjacency_kernel(const uint32_t *adj, int n, int nw,
+                                                        int step, int rows, int cap,
+                                                        uint16_t *edge, uint32_t *row, int *sym) {
+  if (bid_x() < rows)
+    count_symmetry(bid_x(), adj, n, nw, step, sym);
+  else
+    list_edges(bid_x() - rows, adj, n, nw, cap, edge, row, sym + 2);
+}
+
 struct SparseBfsSmem {
   alignas(16) uint16_t edge[SL_E];
   uint32_t row[SL_N];
@@ -427,18 +440,12 @@ struct SparseBfsSmem {
   int reached;
 };
 
-// Workgroup k searches from vertex k * n / 8, as bfs() does, when the edge lists
-// hold the graph (*total <= cap).
-__global__ __launch_bounds__(SB_T) void bfs_sources_sparse_kernel(const uint16_t *edge,
-                                                                   const uint32_t *row, int n,
-                                                                   int cap, const int *total,
-                                                                   int *res) {
-  __shared__ SparseBfsSmem sm;
+// The search from src over `edges` listed edges.
+__device__ __forceinline__ void bfs_sparse(SparseBfsSmem &sm, const uint16_t *edge,
+                                           const uint32_t *row, int n, int edges, int src,
+                                           int *out) {
   static_assert(SL_N % SB_T == 0 && SL_NW == 128, "four vertices a thread, two waves of words");
-  const int edges = *total;
-  if (edges > cap) return;
   const int t = tid_x(), lane = t % 64;
-  const int src = (int)((int64_t)bid_x() * n / NSRC);
   const uint4 *from = reinterpret_cast<const uint4 *>(edge);  // cap is a multiple of 8
   for (int i = t; i < (edges + 7) / 8; i += SB_T) reinterpret_cast<uint4 *>(sm.edge)[i] = from[i];
   for (int v = t; v < n; v += SB_T) sm.row[v] = row[v];
@@ -482,26 +489,50 @@ __global__ __launch_bounds__(SB_T) void bfs_sources_sparse_kernel(const uint16_t
   if (t < SL_NW) atomicAdd(&sm.reached, __popc(sm.visited[t]));
   __syncthreads();
   if (t == 0) {
-    int *out = res + 3 * bid_x();
     out[0] = depth;
     out[1] = sm.reached;
     out[2] = far;
   }
 }
 
-// Feature searches: workgroup k searches from vertex k * n / 8, unless the
-// sparse form has (edges set and *edges <= cap).
+// Feature searches, 1024 < n <= 4096: workgroup k searches from vertex k * n / 8,
+// over the edge lists when they hold the graph (*total <= cap), else over the
+// adjacency rows, whose vertex lists then take the edge lists' place.  One launch
+// for both, and 1024 threads for the rows too, whose loads are what that form
+// waits for: all features of a random graph with n = 1025 and half of all edges
+// 86 -> 59 us, n = 4096 and 2% of them 710 -> 273.
+__global__ __launch_bounds__(SB_T) void bfs_sources_mid_kernel(const uint32_t *adj, int n, int nw,
+                                                               int *lists, const uint16_t *edge,
+                                                               const uint32_t *row, int cap,
+                                                               const int *total, int *res) {
+  __shared__ union {
+    SparseBfsSmem sparse;
+    struct {
+      uint32_t visited[SL_NW], red[SB_T];
+      int cnt[3];
+    } rows;
+  } sm;
+  const int k = bid_x(), edges = *total;
+  const int src = (int)((int64_t)k * n / NSRC);
+  if (edges <= cap) {
+    bfs_sparse(sm.sparse, edge, row, n, edges, src, res + 3 * k);
+  } else {
+    int *cur = lists + (int64_t)k * 2 * n;
+    bfs<SB_T>(adj, n, nw, src, cur, cur + n, nullptr, res + 3 * k, sm.rows.visited, sm.rows.red,
+              sm.rows.cnt);
+  }
+}
+
+// Feature searches, larger n.
 __global__ __launch_bounds__(BFS_T) void bfs_sources_kernel(const uint32_t *adj, int n, int nw,
-                                                            int *lists, int *res,
-                                                            const int *edges, int cap) {
+                                                            int *lists, int *res) {
   __shared__ uint32_t visited[BFS_T * BFS_W];
   __shared__ uint32_t red[BFS_T];
   __shared__ int s_cnt[3];
-  if (edges && *edges <= cap) return;
   const int k = bid_x();
   const int src = (int)((int64_t)k * n / NSRC);
   int *cur = lists + (int64_t)k * 2 * n;
-  bfs(adj, n, nw, src, cur, cur + n, nullptr, res + 3 * k, visited, red, s_cnt);
+  bfs<BFS_T>(adj, n, nw, src, cur, cur + n, nullptr, res + 3 * k, visited, red, s_cnt);
 }
 
 // Vertex levels for the order: the search from the lowest-numbered vertex of
@@ -518,10 +549,10 @@ __global__ __launch_bounds__(BFS_T) void bfs_levels_kernel(const uint32_t *adj, 
   if (far) {
     src = *far;
   } else {
-    bfs(adj, n, nw, 0, lists, lists + n, nullptr, res, visited, red, s_cnt);
+    bfs<BFS_T>(adj, n, nw, 0, lists, lists + n, nullptr, res, visited, red, s_cnt);
     src = res[2];
   }
-  bfs(adj, n, nw, src, lists, lists + n, level, res + 3, visited, red, s_cnt);
+  bfs<BFS_T>(adj, n, nw, src, lists, lists + n, level, res + 3, visited, red, s_cnt);
 }
 
 // The 24 features (one workgroup; fixed-order reductions in double).
@@ -766,7 +797,7 @@ FeatLayout feat_layout(int n) {
   const int nw = (n + 31) / 32;
   L.rstats = take((size_t)n * RS * sizeof(double));
   L.indeg = take((size_t)n * sizeof(int));
-  L.sym = take(3 * sizeof(int));  // two counts of symmetry_kernel, edge_list_kernel's
+  L.sym = take(3 * sizeof(int));  // count_symmetry's two, list_edges' one
   L.adj = take((size_t)n * nw * sizeof(uint32_t));
   L.lists = take((size_t)NSRC * 2 * n * sizeof(int));
   L.res = take((3 * NSRC + 6) * sizeof(int));
@@ -802,20 +833,21 @@ hipError_t launch_graph_features(int op, int n, const float *X, int64_t ld, int 
   in_degree_kernel<<<dim3((n + 255) / 256, (n + chunk - 1) / chunk), dim3(256), 0, s>>>(
       X, ld, n, chunk, indeg);
   const int step = std::max(1, n / 256);
-  symmetry_kernel<<<dim3((n + step - 1) / step), dim3(256), 0, s>>>(adj, n, nw, step, sym);
+  const int rows = (n + step - 1) / step, cap = sparse_cap(n);
+  const bool mid = nw > SB_NW && n <= SL_N;
+  uint16_t *edge = reinterpret_cast<uint16_t *>(lists);
+  uint32_t *row = reinterpret_cast<uint32_t *>(edge + cap);
+  adjacency_kernel<<<dim3(rows + (mid ? (n + 3) / 4 : 0)), dim3(256), 0, s>>>(
+      adj, n, nw, step, rows, cap, edge, row, sym);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (nw <= SB_NW) {
     bfs_sources_small_kernel<<<dim3(NSRC), dim3(SB_T), 0, s>>>(adj, n, nw, res);
-  } else if (n <= SL_N) {
-    const int cap = sparse_cap(n);
-    uint16_t *edge = reinterpret_cast<uint16_t *>(lists);
-    uint32_t *row = reinterpret_cast<uint32_t *>(edge + cap);
-    edge_list_kernel<<<dim3((n + 3) / 4), dim3(256), 0, s>>>(adj, n, nw, cap, edge, row, sym + 2);
-    bfs_sources_sparse_kernel<<<dim3(NSRC), dim3(SB_T), 0, s>>>(edge, row, n, cap, sym + 2, res);
-    bfs_sources_kernel<<<dim3(NSRC), dim3(BFS_T), 0, s>>>(adj, n, nw, lists, res, sym + 2, cap);
+  } else if (mid) {
+    bfs_sources_mid_kernel<<<dim3(NSRC), dim3(SB_T), 0, s>>>(adj, n, nw, lists, edge, row, cap,
+                                                             sym + 2, res);
   } else {
-    bfs_sources_kernel<<<dim3(NSRC), dim3(BFS_T), 0, s>>>(adj, n, nw, lists, res, nullptr, 0);
+    bfs_sources_kernel<<<dim3(NSRC), dim3(BFS_T), 0, s>>>(adj, n, nw, lists, res);
   }
   const int max_based = (op == 2 || op == 3 || op == 4) ? 1 : 0;
   features_kernel<<<dim3(1), dim3(256), 0, s>>>(rstats, indeg, sym, res, n, max_based, epi, f,

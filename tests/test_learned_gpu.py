@@ -170,3 +170,14 @@ def test_sparse_searches_match_oracle(gpu, oracle_learned, n, kind):
     f = LG.graph_features("min_plus", X, True).cpu().numpy()
     fo = oracle_learned.graph_features("min_plus", X.cpu().numpy(), True)
     np.testing.assert_allclose(f, fo, rtol=2e-6, atol=1e-7)
+
+
+@pytest.mark.parametrize("n,p", [(1025, 0.05), (1025, 0.5), (2050, 0.3), (4096, 0.01), (4096, 0.0002)])
+def test_searches_of_dense_and_cut_graphs_match_oracle(gpu, oracle_learned, n, p):
+    """Too many edges for the lists (adjacency rows, all threads of the same
+    kernel), and at the last one so few that most vertices are not reached."""
+    X = er_family(gpu, "min_plus", n, p, 5)
+    print("searches", n, p, flush=True)
+    f = LG.graph_features("min_plus", X, True).cpu().numpy()
+    fo = oracle_learned.graph_features("min_plus", X.cpu().numpy(), True)
+    np.testing.assert_allclose(f, fo, rtol=2e-6, atol=1e-7)
