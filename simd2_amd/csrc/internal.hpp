@@ -219,7 +219,7 @@ struct SchedArgs {
                       //   mirrored pair, if the tiles are square
   int rows_limit, changed_limit;
   int rows_auto, changed_auto;
-  int square;         // the tile shape is square
+  float mirror_cost;  // cost of a tile of a symmetric matrix against one of another
   float cost_slab_tile, cost_row_entry, cost_changed_entry, cost_list;
   unsigned long long *work;
   int *sq_mode;

@@ -385,7 +385,7 @@ __global__ __launch_bounds__(SCAN_T) void list_scan_kernel(SchedArgs a) {
       // symmetric: row passes over the changed entries, then a symmetrising pass
       const double c_sym = (double)tc * a.cost_row_entry + 2.0 * a.cost_list;
       // the tiled kernel computes one tile of each mirrored pair (square tiles)
-      double best = (double)*a.work * a.cost_slab_tile * (sym && a.square ? 0.5 : 1.0);
+      double best = (double)*a.work * a.cost_slab_tile * (sym ? a.mirror_cost : 1.0f);
       if (rows_ok && c_rows < best) {
         mode = 1;
         best = c_rows;

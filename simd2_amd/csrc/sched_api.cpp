@@ -184,6 +184,13 @@ int simd2_converge_scheduled(int op, int n, float *X, int ldx, int do_epilogue,
   // The check takes 5 us, 37 at n = 4096.
   const bool sym_on = changed_on || (ci.bm == ci.bn && L.tiles_r * L.tiles_c > device_cu_count());
   if (e == hipSuccess && sym_on) e = launch_sched_symmetry(buf[0], L.P, n, asym, stream);
+  // What half of the tiles saves: with more than a CU holds at once (8 of 64x64)
+  // the next ones even the CUs out; up to there all start together, and the CU
+  // that is left with most of its own decides (a dense squaring, symmetric / not,
+  // us: n = 1500 145 / 150, 2000 192 / 254, 2500 500 / 531; 3000 538 / 772, 3700
+  // 915 / 1412, 4096 1031 / 1738).
+  const float mirror_cost =
+      ci.bm == ci.bn && L.tiles_r * L.tiles_c > 8 * device_cu_count() ? 0.65f : 1.0f;
   if (e == hipSuccess)
     e = launch_sched_occupancy(op, cfg, buf[0], L.P, n, L.tiles_r, L.tiles_c, L.slabs, xocc[0],
                                yocc[0], nullptr, stream);
@@ -226,7 +233,7 @@ int simd2_converge_scheduled(int op, int n, float *X, int ldx, int do_epilogue,
       a.changed_limit = a.prev ? changed_per_row * n : 0;
       a.rows_auto = rows_auto ? 1 : 0;
       a.changed_auto = changed_auto ? 1 : 0;
-      a.square = ci.bm == ci.bn;
+      a.mirror_cost = mirror_cost;
       a.cost_slab_tile = (float)(16.0 * ci.bm * ci.bn * ps_term);
       a.cost_list = (float)((double)n * n * PS_LIST_ELEM);
       a.cost_row_entry = (float)(n * PS_ROW_ENTRY_COL);
