@@ -26,6 +26,7 @@
 // conversion per term took 811 and 6390.
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "internal.hpp"
@@ -336,30 +337,45 @@ __global__ __launch_bounds__(256 * G) void tensor_emu_kernel(
   }
 }
 
-// The sums on a 16x16 tile, one output a thread: for the fewest outputs, where
-// the length of a thread's chain counts and not the instructions.
+// A 16x16 tile, one output a thread, any alignment: for the fewest outputs,
+// where the length of a thread's chain counts and not the instructions, and for
+// the shortest K, which the slabs of the tiles above would mostly pad.
 constexpr int TE = 16;
 
+template <int OP> __device__ __forceinline__ float emu_step(float acc, __half x, __half y) {
+  constexpr int t = Emu<OP>::term, f = Emu<OP>::fold;
+  if constexpr (OP == 7)
+    return (float)(acc > 0.f || (__half2float(x) > 0.f && __half2float(y) > 0.f));
+  __half r;
+  if constexpr (t == emu_add) r = __hadd(x, y);
+  if constexpr (t == emu_mul) r = __hmul(x, y);
+  if constexpr (t == emu_min) r = __hmin(x, y);
+  if constexpr (t == emu_max) r = __hmax(x, y);
+  if constexpr (t == emu_sub2) {
+    r = __hsub(x, y);
+    r = __hmul(r, r);
+  }
+  const float v = __half2float(r);
+  return f == 0 ? fminf(acc, v) : f == 1 ? fmaxf(acc, v) : acc + v;
+}
+
 template <int OP>
-__global__ __launch_bounds__(256) void tensor_emu_sum16_kernel(const __half *__restrict__ a,
-                                                               const __half *__restrict__ b,
-                                                               const float *c, float *d, int m,
-                                                               int n, int k, int do_epilogue) {
+__global__ __launch_bounds__(256) void tensor_emu16_kernel(const __half *__restrict__ a,
+                                                           const __half *__restrict__ b,
+                                                           const float *c, float *d, int m, int n,
+                                                           int k, int do_epilogue) {
   __shared__ __half As[TE][TE + 2];
   __shared__ __half Bs[TE][TE + 2];
   const int tx = tid_x() % TE;   // column within the tile
   const int ty = tid_x() / TE;   // row within the tile
   const int row0 = bid_y() * TE, col0 = bid_x() * TE;
-  float acc = 0.f;
+  float acc = Emu<OP>::fold == 0 ? __builtin_inff() : 0.f;
   for (int k0 = 0; k0 < k; k0 += TE) {
     As[ty][tx] = a[(int64_t)(row0 + ty) * k + k0 + tx];
     Bs[ty][tx] = b[(int64_t)(k0 + ty) * n + col0 + tx];
     __syncthreads();
 #pragma unroll
-    for (int kk = 0; kk < TE; ++kk) {
-      const __half x = As[ty][kk], y = Bs[kk][tx], f = OP == 8 ? __hsub(x, y) : x;
-      acc += __half2float(__hmul(f, OP == 8 ? f : y));
-    }
+    for (int kk = 0; kk < TE; ++kk) acc = emu_step<OP>(acc, As[ty][kk], Bs[kk][tx]);
     __syncthreads();
   }
   const int64_t idx = (int64_t)(row0 + ty) * n + col0 + tx;
@@ -374,38 +390,78 @@ void launch_emu_tiles(const __half *a, const __half *b, const float *c, float *d
       a, b, c, d, m, n, k, do_epilogue, tiles_c);
 }
 
+// Where a 16x16 tile with one output a thread takes no longer than the tiles (us,
+// one output a thread / best tile): few outputs, up to `most` 16x16 tiles per CU;
+// more for K below a slab of the 32x32 tiles (64) or just past one, which those
+// pad.  min_plus 512^2 of K = 16: 2.8 / 4.6, 64: 4.8 / 4.7, 128: 7.5 / 6.0; plus_mul
+// 800^2 of K = 16: 3.7 / 5.8, 80: 8.4 / 8.7, 128: 11.9 / 8.8.  Sums cannot split
+// K, so they keep it at any K (minus_square 320^2 of K = 1024 27.6 / 32.0, 16x2048
+// 26.8 / 31.9) unless B leaves the L2 (4 MiB: 48x4096 of K = 1024 39.8 / 32.2).
+// Where the operands are not 16-byte aligned the 64x64 tiles load element by
+// element (minus_square 640^2 of K = 256: 16.7 / 28.4, min_plus 15.7 / 19.6) and
+// pay for whole tiles (16x65536 of K = 128: 18.8 / 37.4).
+template <int OP> bool one_output_a_thread(bool aligned, int64_t m, int64_t n, int64_t k) {
+  constexpr bool SUM = Emu<OP>::fold == 2, SQUARES = Emu<OP>::term == emu_sub2;
+  const int64_t cus = device_cu_count(), tiles = m / TE * (n / TE);
+  if (m / TE > 65535) return false;  // the grid's second dimension
+  const bool thin = std::min(m, n) == TE;  // 32x32 tiles would be half empty
+  double most;
+  if (!aligned) {
+    if (std::min(m, n) < 64) return true;
+    most = k <= 16   ? 40
+           : k <= 32 ? (SUM ? 36 : 25)
+           : k <= 48 ? (SUM ? 30 : 16)
+                     : k <= 128 ? (SUM ? 16 : 12) : (SUM ? 12 : 8);
+  } else {
+    most = k <= 16 ? 36 : k <= 48 ? 10 : k <= 96 ? 4.5 : k <= 128 ? 2.5 : 0;
+    if (k > 128 && k <= 176) most = SUM ? 4.2 : 3.5;  // three slabs of 64
+    if (SUM && k > 64 && k <= 80) most = 10;
+    if (SUM && k > 176 && k * n <= 1 << 21) most = 2;
+    if (SQUARES && k > 80) most *= k > 176 ? 1.5 : 2;
+    if (SQUARES && thin && tiles >= 4 * cus) return true;
+    if (thin) most *= 2;
+  }
+  return tiles <= most * cus;
+}
+
 template <int OP>
 void launch_emu_op(const __half *a, const __half *b, const float *c, float *d, int m, int n, int k,
                    int do_epilogue, hipStream_t s) {
   auto aligned = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+  const bool vec = aligned(a) && aligned(b) && aligned(d) && (!do_epilogue || aligned(c));
   const int64_t cus = device_cu_count();
+  const int64_t t32 = (int64_t)((m + 31) / 32) * ((n + 31) / 32);
   const int64_t t64 = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
   const int64_t t128 = (int64_t)((m + 127) / 128) * ((n + 127) / 128);
   using Large = EmuTile<128, 8>;
   using Mid = EmuTile<64, 4>;
   using Small = EmuTile<32, 2>;
-  if (!aligned(a) || !aligned(b) || !aligned(d) || (do_epilogue && !aligned(c)))
-    return launch_emu_tiles<OP, Mid, 1, false>(a, b, c, d, m, n, k, do_epilogue, s);
+  if (one_output_a_thread<OP>(vec, m, n, k)) {
+    tensor_emu16_kernel<OP><<<dim3(n / TE, m / TE), dim3(256), 0, s>>>(a, b, c, d, m, n, k,
+                                                                       do_epilogue);
+    return;
+  }
+  if (!vec) return launch_emu_tiles<OP, Mid, 1, false>(a, b, c, d, m, n, k, do_epilogue, s);
+  const bool thin = std::min(m, n) <= 32;  // larger tiles would be half empty
   // 128x128 tiles from two per CU up (min_plus 4096^3 1549 us; one per CU, at
   // 2048^3, loses: 296 us against 228 in 64x64).
-  if (t128 >= 2 * cus)
+  if (t128 >= 2 * cus && std::min(m, n) > 64)
     return launch_emu_tiles<OP, Large, 1, true>(a, b, c, d, m, n, k, do_epilogue, s);
   if constexpr (Emu<OP>::fold == 2) {
-    // Sums cannot split K: one output a thread below 512^2 outputs (256^3
-    // plus_mul 7.7 us, 8.6 in 32x32 tiles; 512^3 21 and 15), then 32x32 tiles
-    // (1296^3 125 us, 150 in 64x64) unless K is too short to pay for them.
-    if (t64 * 16 <= cus) {
-      tensor_emu_sum16_kernel<OP><<<dim3(n / TE, m / TE), dim3(256), 0, s>>>(a, b, c, d, m, n, k,
-                                                                             do_epilogue);
-      return;
-    }
-    if (k >= 128) return launch_emu_tiles<OP, Small, 1, true>(a, b, c, d, m, n, k, do_epilogue, s);
+    // Sums cannot split K: 32x32 tiles (1296^3 125 us, 150 in 64x64; 640^2 of K =
+    // 64 4.9 and 7.9) unless K is short, or fills its last 64-k slab badly and the
+    // 64x64 tiles are many (1280^2 of K = 96 15.4 and 14.6).
+    if (thin || k >= 128 ||
+        (k >= 48 && (k % 64 == 0 || k % 64 >= 48 || t64 < cus)))
+      return launch_emu_tiles<OP, Small, 1, true>(a, b, c, d, m, n, k, do_epilogue, s);
   } else {
     // Few tiles: 32x32 ones below 1024^2 / 2 outputs (512^3 9 us, 18 in 64x64;
-    // 1040x784x304 24 and 15.5), K in four parts when it has four slabs.
-    if (t64 * 2 < cus && k >= 256)
+    // 1040x784x304 24 and 15.5), twice as many for a K that is not worth splitting
+    // (800^2 of K = 64 5.6, 9.0 in 64x64), and of thin products (16x8192 of K = 1024 14.8,
+    // 32.8 in 64x64), K in four parts when it has four slabs.
+    if (t32 <= 2 * cus && k >= 256)
       return launch_emu_tiles<OP, Small, 4, true>(a, b, c, d, m, n, k, do_epilogue, s);
-    if (t64 * 2 < cus)
+    if (thin || t32 <= (k < 256 ? 4 : 2) * cus)
       return launch_emu_tiles<OP, Small, 1, true>(a, b, c, d, m, n, k, do_epilogue, s);
     if (t64 < 2 * cus && k >= 128)
       return launch_emu_tiles<OP, Mid, 4, true>(a, b, c, d, m, n, k, do_epilogue, s);
