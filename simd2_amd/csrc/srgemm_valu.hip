@@ -359,15 +359,23 @@ ValuCfgInfo valu_cfg_info(int cfg) {
   return {CfgL::BM, CfgL::BN, CfgL::BK, 256};
 }
 
-// Tile shape choice, measured on MI355X for square problems (n = 1024 .. 8192,
-// min_plus / max_min / minus_square, us in 64x64, 128x64 and 128x128 tiles for
-// min_plus): the 64x64 tiles' many workgroups waste least of a last round
-// (3328: 965, 1058, 1181; 4608: 2451, 2570, 2891; 5120: 3260, 3337, 3663; 7168:
-// 8788, 8782, 9090); the 128x128 tiles read LDS least and win where their own
-// rounds fill (6144: 5558, 5407, 5479, three rounds; 8192: 12893, 12620,
-// 12588; minus_square 16384^2 x 128: 1432, 1384, 1310).  At 4096 all three
-// agree within 2% and the 128x64 tiles, two full rounds, are kept.  Shapes the
-// autotuner has timed (simd2_autotune) use the recorded winner instead.
+// Tile shape choice, measured on MI355X (us in 64x64, 128x64 and 128x128 tiles).
+// What a size wastes is its last round over the CUs.  The 64x64 tiles' many
+// workgroups waste least (min_plus 3328^3: 965, 1058, 1181; 4608: 2451, 2570,
+// 2891; 5120: 3260, 3337, 3663).  The larger tiles read LDS less and win where
+// their rounds fill:
+//   * minus_square, whose step is one instruction shorter, in 128x128 tiles from
+//     more than three per CU up (4096^2 x 1024: 699, 672, 651; 8192x4096x1000
+//     1317, 1290, 1244; 5376^2 x 300 358, 350, 340; rounds not full: 4608^2 x 300
+//     269, 274, 286; 5120^2 x 300 322, 329, 333);
+//   * the others in 128x128 tiles from 5900^2 up, where three per CU at once fill
+//     (6144^3: 5558, 5407, 5479; 8192: 12893, 12620, 12588; not full: 7168: 8788,
+//     8782, 9090), and in 128x64 tiles at eight and more full rounds up to 4096^2
+//     (max_mul 4096^3 1718, 1699, 1759; min_plus within 1%; not full: 3900^2 x 512
+//     208, 225, 236; 4100^2 x 512 235, 245, 281).  Above, those gain 1 to 3% again at
+//     some sizes, but the scheduled loop, which asks here too, can halve the work of
+//     square tiles only.
+// Shapes the autotuner has timed (simd2_autotune) use the recorded winner instead.
 namespace {
 struct TunedEntry { int op, R, Cn, K, cfg; };
 constexpr int TUNED_MAX = 64;
@@ -394,11 +402,21 @@ int valu_pick_cfg(int op, int R, int Cn, int K) {
       if (g_tuned[i].op == op && g_tuned[i].R == R && g_tuned[i].Cn == Cn && g_tuned[i].K == K)
         return g_tuned[i].cfg;
   }
+  const int64_t cus = device_cu_count();
   const double area = (double)R * Cn;
-  const double scale = 256.0 / device_cu_count();   // rule is for 256 CUs
-  const double a = area * scale;
-  if (a <= 4096.0 * 4096.0 * 1.01) return a > 3840.0 * 3840.0 ? CFG_M128x64 : CFG_S64;
-  const double rounds = (double)((R + 127) / 128) * ((Cn + 127) / 128) / (3 * device_cu_count());
+  const double a = area * (256.0 / cus);   // rule is for 256 CUs
+  auto tiles = [&](int bm, int bn) {
+    return (int64_t)((R + bm - 1) / bm) * ((Cn + bn - 1) / bn);
+  };
+  // share of the CUs' rounds that ends up as outputs
+  auto fill = [&](int bm, int bn) {
+    const int64_t rounds = (tiles(bm, bn) + cus - 1) / cus;
+    return area / ((double)bm * bn * cus * rounds);
+  };
+  if (op == 8 && tiles(128, 128) > 3 * cus && fill(128, 128) >= 0.91) return CFG_L128;
+  if (a <= 4096.0 * 4096.0 * 1.01)
+    return tiles(128, 64) >= 8 * cus && fill(128, 64) >= 0.975 ? CFG_M128x64 : CFG_S64;
+  const double rounds = (double)tiles(128, 128) / (3 * cus);
   return a >= 5900.0 * 5900.0 && rounds >= 0.85 * ceil(rounds) ? CFG_L128 : CFG_S64;
 }
 

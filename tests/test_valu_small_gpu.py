@@ -93,3 +93,15 @@ def test_loop_uses_the_change_test(n):
     Z, itr_r, st_r = simd2_amd.converge("min_plus", torch.from_numpy(X).cuda(),
                                         check="threshold", flags=simd2_amd.CONVERGE_REFERENCE)
     assert (st, itr) == (0, itr_r) and st_r == 0 and torch.equal(Y, Z)
+
+
+@pytest.mark.parametrize("op,m,n,k,cfg", [
+    ("minus_square", 8192, 4096, 300, 0), ("minus_square", 5376, 5376, 300, 0),
+    ("minus_square", 4608, 4608, 300, 1), ("minus_square", 5120, 5120, 128, 1),
+    ("min_plus", 3900, 3900, 512, 1), ("min_plus", 4096, 4096, 4096, 2),
+    ("max_min", 2048, 8192, 1000, 2), ("max_min", 4100, 4100, 300, 1)])
+def test_tile_shape_by_full_rounds(op, m, n, k, cfg):
+    """The shape that was fastest there (256 CUs; others round elsewhere)."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("measured with 256 CUs")
+    assert simd2_amd.lib().simd2_pick_tile_config(simd2_amd.OPS.index(op), n, m, k) == cfg
