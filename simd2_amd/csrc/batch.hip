@@ -56,7 +56,7 @@ __attribute__((amdgpu_waves_per_eu(Cfg::WAVES))) void batch_valu_kernel(
   float *nxt = pool + (parity ? G.off[0] : G.off[1]);
   const Epilogue e{G.epi ? cur : nullptr, G.ld, cur, G.ld, changed + g, nullptr, G.mode};
   const int tr = tile >> 16, tc = tile & 0xffff;
-  valu_tile<Op, Cfg::BM, Cfg::BN, Cfg::TM, Cfg::TN, Cfg::BK, false, true>(
+  valu_tile<Op, Cfg::BM, Cfg::BN, Cfg::TM, Cfg::TN, Cfg::BK, true>(
       G.n, G.n, G.kpad, cur, G.ld, cur, G.ld, nxt, G.ld, e, tr * Cfg::BM, tc * Cfg::BN,
       nullptr, sm);
 }

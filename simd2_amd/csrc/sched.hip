@@ -108,7 +108,7 @@ __attribute__((amdgpu_waves_per_eu(G > 1 ? 1 : Cfg::WAVES))) void sched_kernel(S
 
   float acc[TM][TN];
   if constexpr (G == 1) {
-    valu_mainloop<Op, BM, BN, TM, TN, BK, false, true>(a.n, a.n, a.kpad, a.cur, a.ld, a.cur,
+    valu_mainloop<Op, BM, BN, TM, TN, BK, true>(a.n, a.n, a.kpad, a.cur, a.ld, a.cur,
                                                        a.ld, row0, col0, list, nlist, sm, acc);
   } else {
     // group g: entries [b, b + c) of the list, padded to `steps` by repeats
@@ -118,7 +118,7 @@ __attribute__((amdgpu_waves_per_eu(G > 1 ? 1 : Cfg::WAVES))) void sched_kernel(S
     for (int i = tid; i < steps; i += NT)
       glist[grp][i] = list[c > 0 ? b + min(i, c - 1) : 0];
     __syncthreads();
-    valu_mainloop<Op, BM, BN, TM, TN, BK, false, true>(a.n, a.n, a.kpad, a.cur, a.ld, a.cur,
+    valu_mainloop<Op, BM, BN, TM, TN, BK, true>(a.n, a.n, a.kpad, a.cur, a.ld, a.cur,
                                                        a.ld, row0, col0, glist[grp], steps, sm,
                                                        acc, tid);
     // the main loop ends with a barrier after every read of the slabs

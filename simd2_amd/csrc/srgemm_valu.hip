@@ -50,10 +50,10 @@ __attribute__((amdgpu_waves_per_eu(WAVES))) void srgemm_valu_kernel(
   int *flag = e.tile_flags ? &e.tile_flags[tr * tiles_c + tc] : nullptr;
   const int row0 = tr * BM, col0 = tc * BN;
   if (!OFFGRID || (row0 + BM <= R && col0 + BN <= Cn))
-    valu_tile<Op, BM, BN, TM, TN, BK, false, false, OFFGRID>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e,
+    valu_tile<Op, BM, BN, TM, TN, BK, false, OFFGRID>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e,
                                                              row0, col0, flag, sm);
   else
-    valu_tile<Op, BM, BN, TM, TN, BK, false, true, true, true>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e,
+    valu_tile<Op, BM, BN, TM, TN, BK, true, true, true>(R, Cn, K, X, ldx, Y, ldy, O, ldo, e,
                                                                row0, col0, flag, sm);
 }
 
@@ -147,14 +147,9 @@ __device__ __forceinline__ void wave_loop(WaveSmem &sm, float (&acc)[WTM][WTM],
 #pragma unroll
       for (int i = 0; i < WTM; ++i)
 #pragma unroll
-        for (int j = 0; j < WTM; ++j) {
-          if constexpr (is_fused<Op>::value)
-            acc[i][j] = Op::fma_step(Op::fma_step(acc[i][j], a[s][0][i], b[s][0][j]), a[s][1][i],
-                                     b[s][1][j]);
-          else
-            acc[i][j] = Op::add3(acc[i][j], Op::mul(a[s][0][i], b[s][0][j]),
-                                 Op::mul(a[s][1][i], b[s][1][j]));
-        }
+        for (int j = 0; j < WTM; ++j)
+          acc[i][j] = Op::add3(acc[i][j], Op::mul(a[s][0][i], b[s][0][j]),
+                               Op::mul(a[s][1][i], b[s][1][j]));
     }
   }
 }
@@ -253,10 +248,10 @@ __global__ __launch_bounds__(256 * SK_GROUPS) void srgemm_valu_splitk_kernel(
   const int per = ((K + S::BK - 1) / S::BK + SK_GROUPS - 1) / SK_GROUPS;
   float acc[S::TM][S::TN];
   if (!RAGGED || (row0 + S::BM <= R && col0 + S::BN <= Cn))
-    valu_mainloop<Op, S::BM, S::BN, S::TM, S::TN, S::BK, false, false, RAGGED>(
+    valu_mainloop<Op, S::BM, S::BN, S::TM, S::TN, S::BK, false, RAGGED>(
         R, Cn, K, X, ldx, Y, ldy, row0, col0, nullptr, 0, sm[g], acc, t, g * per, (g + 1) * per);
   else
-    valu_mainloop<Op, S::BM, S::BN, S::TM, S::TN, S::BK, false, false, true, true>(
+    valu_mainloop<Op, S::BM, S::BN, S::TM, S::TN, S::BK, false, true, true>(
         R, Cn, K, X, ldx, Y, ldy, row0, col0, nullptr, 0, sm[g], acc, t, g * per, (g + 1) * per);
   // The main loop ends with a barrier after every read of the slabs: groups
   // 1.. park their partial tiles in their own LDS (16 KB of its 16.5).
@@ -281,7 +276,7 @@ __global__ __launch_bounds__(256 * SK_GROUPS) void srgemm_valu_splitk_kernel(
           acc[i][j] = Op::add(acc[i][j], part[(i * S::TN + j) * 256 + t]);
     }
   }
-  valu_epilogue<Op, S::BM, S::BN, S::TM, S::TN, false, RAGGED>(R, Cn, O, ldo, e, row0, col0,
+  valu_epilogue<Op, S::BM, S::BN, S::TM, S::TN, RAGGED>(R, Cn, O, ldo, e, row0, col0,
                                                                flag, &sm[0].changed, acc, t,
                                                                g == 0);
 }

@@ -65,19 +65,18 @@ __device__ __forceinline__ void load_slab_form(vf4 (&xv)[BM * BK / 4 / NT],
                                                int k0, int tid);
 
 // KT: K may end inside a slab -- that slab (uniform over the workgroup) takes
-// the checked form, the others the fast one.  GUARD (with the fast form): the
+// the checked form, the others the fast one.  GUARD (of the fast form): the
 // tile may reach past row R or column Cn; a 4-float load wholly inside the
 // matrix stays one 128-bit load, X rows past R read as padding, and a Y group
 // reaching past Cn is read element by element.
-template <class Op, int BM, int BN, int BK, int NT, bool CHECKED, bool KT = false,
-          bool GUARD = false>
+template <class Op, int BM, int BN, int BK, int NT, bool KT = false, bool GUARD = false>
 __device__ __forceinline__ void load_slab(vf4 (&xv)[BM * BK / 4 / NT],
                                           vf4 (&yv)[BK * BN / 4 / NT],
                                           const float *__restrict__ X, int64_t ldx,
                                           const float *__restrict__ Y, int64_t ldy,
                                           int R, int Cn, int K, int row0, int col0,
                                           int k0, int tid) {
-  if (CHECKED || (KT && k0 + BK > K))
+  if (KT && k0 + BK > K)
     load_slab_form<Op, BM, BN, BK, NT, true>(xv, yv, X, ldx, Y, ldy, R, Cn, K, row0, col0, k0,
                                              tid);
   else
@@ -160,8 +159,8 @@ __device__ __forceinline__ void store_slab(float (*Xs)[XLD], float (*Ys)[BN],
   }
 }
 
-// LDS of one workgroup of the VALU kernel (shared by the fast and checked
-// tile bodies when a kernel contains both).
+// LDS of one workgroup of the VALU kernel (shared by the tile bodies when a
+// kernel contains several).
 template <int BM, int BN, int BK> struct ValuSmem {
   __attribute__((aligned(16))) float Xs[2][BK][BM + 4];
   __attribute__((aligned(16))) float Ys[2][BK][BN];
@@ -172,8 +171,8 @@ template <int BM, int BN, int BK> struct ValuSmem {
 // the K slabs, double-buffered through LDS.  LIST: only the BK-deep slabs
 // whose indices are list[0 .. nlist) (ascending, in LDS) are visited -- the
 // others are known to hold only the (+)-identity and contribute nothing.
-template <class Op, int BM, int BN, int TM, int TN, int BK, bool CHECKED, bool LIST,
-          bool KT = false, bool GUARD = false>
+template <class Op, int BM, int BN, int TM, int TN, int BK, bool LIST, bool KT = false,
+          bool GUARD = false>
 __device__ __forceinline__ void valu_mainloop(int R, int Cn, int K, const float *__restrict__ X,
                                               int64_t ldx, const float *__restrict__ Y,
                                               int64_t ldy, int row0, int col0,
@@ -206,8 +205,8 @@ __device__ __forceinline__ void valu_mainloop(int R, int Cn, int K, const float 
   const int nkt = LIST ? nlist : kt_end >= 0 ? kt_end - kt_begin : (K + BK - 1) / BK;
   if (nkt > 0) {
     const int k0 = (LIST ? (int)list[0] : kt_begin) * BK;
-    load_slab<Op, BM, BN, BK, NT, CHECKED, KT, GUARD>(xv, yv, X, ldx, Y, ldy, R, Cn, K, row0,
-                                                      col0, k0, tid);
+    load_slab<Op, BM, BN, BK, NT, KT, GUARD>(xv, yv, X, ldx, Y, ldy, R, Cn, K, row0, col0, k0,
+                                             tid);
     store_slab<BM, BN, BK, NT, XLD>(Xs[0], Ys[0], xv, yv, tid);
   }
   __syncthreads();
@@ -219,8 +218,8 @@ __device__ __forceinline__ void valu_mainloop(int R, int Cn, int K, const float 
     // branch the compiler keeps the prefetch in scratch and waits for it.
     const int kn = kt + 1 < nkt ? kt + 1 : kt;
     const int knext = (LIST ? (int)list[kn] : kt_begin + kn) * BK;
-    load_slab<Op, BM, BN, BK, NT, CHECKED, KT, GUARD>(xv, yv, X, ldx, Y, ldy, R, Cn, K, row0,
-                                                      col0, knext, tid);
+    load_slab<Op, BM, BN, BK, NT, KT, GUARD>(xv, yv, X, ldx, Y, ldy, R, Cn, K, row0, col0, knext,
+                                             tid);
 #pragma unroll
     for (int k = 0; k < BK; k += 2) {
       // Keep each k-pair's LDS reads next to its arithmetic: without this
@@ -257,7 +256,7 @@ __device__ __forceinline__ void valu_mainloop(int R, int Cn, int K, const float 
   }
 }
 
-template <class Op, int BM, int BN, int TM, int TN, bool CHECKED, bool MASKED>
+template <class Op, int BM, int BN, int TM, int TN, bool MASKED>
 __device__ __forceinline__ void valu_epilogue(int R, int Cn, float *O, int64_t ldo,
                                               const Epilogue &e, int row0, int col0,
                                               int *tile_flag, int *changed_slot,
@@ -266,19 +265,17 @@ __device__ __forceinline__ void valu_epilogue(int R, int Cn, float *O, int64_t l
 // One BM x BN output tile at (row0, col0) of the row-major problem; the whole
 // workgroup calls it.  tile_flag, when set, receives 1 / 0 for "some element
 // of this tile changed".
-//   CHECKED: per-element bounds on every load (op padding) and store.
-//   MASKED (with !CHECKED): the operands are stored padded -- every row and
-//     column the tile and the K loop touch exists in memory, and the K
-//     padding holds the op's pad values -- so loads stay 128-bit; only the
-//     epilogue is limited to r < R, c < Cn.
-//   KT (with !CHECKED): K need not be a multiple of BK: the last, partial
-//     slab is loaded checked.
+//   MASKED: the operands are stored padded -- every row and column the tile
+//     and the K loop touch exists in memory, and the K padding holds the op's
+//     pad values -- so loads stay 128-bit; only the epilogue is limited to
+//     r < R, c < Cn.
+//   KT: K need not be a multiple of BK: the last, partial slab is loaded
+//     element by element.
 //   GUARD (with MASKED and KT): the tile reaches past row R or column Cn of
-//     an unpadded matrix whose rows are 16-byte aligned; loads wholly inside
-//     stay 128-bit, the rest are guarded (load_slab), and the epilogue is
-//     MASKED's.
-template <class Op, int BM, int BN, int TM, int TN, int BK, bool CHECKED, bool MASKED = false,
-          bool KT = false, bool GUARD = false>
+//     an unpadded matrix; loads wholly inside stay 128-bit, the rest are
+//     guarded (load_slab), and the epilogue is MASKED's.
+template <class Op, int BM, int BN, int TM, int TN, int BK, bool MASKED = false, bool KT = false,
+          bool GUARD = false>
 __device__ __forceinline__ void valu_tile(int R, int Cn, int K, const float *__restrict__ X,
                                           int64_t ldx, const float *__restrict__ Y, int64_t ldy,
                                           float *O, int64_t ldo, const Epilogue &e, int row0,
@@ -300,14 +297,13 @@ __device__ __forceinline__ void valu_tile(int R, int Cn, int K, const float *__r
   if (tid == 0) sm.changed = 0;
 
   float acc[TM][TN];
-  valu_mainloop<Op, BM, BN, TM, TN, BK, CHECKED, false, KT, GUARD>(R, Cn, K, X, ldx, Y, ldy,
-                                                                    row0, col0, nullptr, 0, sm,
-                                                                    acc);
+  valu_mainloop<Op, BM, BN, TM, TN, BK, false, KT, GUARD>(R, Cn, K, X, ldx, Y, ldy, row0, col0,
+                                                          nullptr, 0, sm, acc);
   (void)XL;
   (void)YL;
   (void)XLD;
-  valu_epilogue<Op, BM, BN, TM, TN, CHECKED, MASKED>(R, Cn, O, ldo, e, row0, col0, tile_flag,
-                                                     &sm.changed, acc, tid, true);
+  valu_epilogue<Op, BM, BN, TM, TN, MASKED>(R, Cn, O, ldo, e, row0, col0, tile_flag, &sm.changed,
+                                            acc, tid, true);
 }
 
 // Epilogue of a BM x BN tile from the thread's acc: (+) C, optional APLP
@@ -315,7 +311,7 @@ __device__ __forceinline__ void valu_tile(int R, int Cn, int K, const float *__r
 // (the flags take a barrier); only threads with `active` set store, tid
 // being their index among the tile's threads.  *changed_slot (LDS) must be
 // cleared before a barrier that precedes this call.
-template <class Op, int BM, int BN, int TM, int TN, bool CHECKED, bool MASKED>
+template <class Op, int BM, int BN, int TM, int TN, bool MASKED>
 __device__ __forceinline__ void valu_epilogue(int R, int Cn, float *O, int64_t ldo,
                                               const Epilogue &e, int row0, int col0,
                                               int *tile_flag, int *changed_slot,
@@ -339,7 +335,7 @@ __device__ __forceinline__ void valu_epilogue(int R, int Cn, float *O, int64_t l
         float v[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] = acc[i][gj * 4 + q];
-        if (!CHECKED && (!MASKED || (r < R && c + 4 <= Cn))) {
+        if (!MASKED || (r < R && c + 4 <= Cn)) {
           if (e.C) {
             const vf4u cv = *reinterpret_cast<const vf4u *>(e.C + (int64_t)r * e.ldc + c);
             v[0] = Op::add(v[0], cv.x); v[1] = Op::add(v[1], cv.y);
