@@ -235,8 +235,8 @@ __global__ __launch_bounds__(WR * WC * 64) void orand_packed_kernel(
   // time, a wave reading whole rows with a slab per lane, and only those with a 1
   // in A are taken: a slab that is merely loaded and converted costs 0.7 us of the
   // 1.0 us of one that is multiplied.  8192^3, every slab taken and here: no bit at
-  // all 187 -> 45 us, blocks of 64 on the diagonal 187 -> 55, density 1e-5 188 ->
-  // 102, 1e-4 204 -> 210, 0.5 266 -> 272 (4096^3 38.3 -> 39).  A loop of its own
+  // all 187 -> 44 us, blocks of 64 on the diagonal 187 -> 54, density 1e-5 188 ->
+  // 103, 1e-4 204 -> 210, 0.5 266 -> 269 (4096^3 38.3 -> 38.5).  A loop of its own
   // for the second part would leave the first as it was, but needs a second set
   // of accumulator registers.
   constexpr int SCAN = 60;  // leaves lanes for the slabs asked for past the last
@@ -292,12 +292,14 @@ __global__ __launch_bounds__(WR * WC * 64) void orand_packed_kernel(
       __syncthreads();
     };
     int s = all && none ? 2 : 0, end = s ? 0 : count;
+    const uint32_t hold = all ? 0u : 1u;  // listed slabs hold a 1 (or padding that may)
     while (s < end) {
       step(s, pre0, kwa);
-      const uint32_t was = now;
+      uint32_t was = now | hold;
       if (s + 1 < count) step(s + 1, pre1, kwb);
       s += 2;
-      end = all && !((was | now) & a_bits) ? 0 : end;
+      was |= now;
+      end = was & a_bits ? end : 0;
     }
     if (end == 0) rest = s;
     for (count = 0; count == 0 && rest < nslab; rest += SCAN) {
