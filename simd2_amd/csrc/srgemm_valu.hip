@@ -362,7 +362,9 @@ ValuCfgInfo valu_cfg_info(int cfg) {
 //   * minus_square, whose step is one instruction shorter, in 128x128 tiles from
 //     more than three per CU up (4096^2 x 1024: 699, 672, 651; 8192x4096x1000
 //     1317, 1290, 1244; 5376^2 x 300 358, 350, 340; rounds not full: 4608^2 x 300
-//     269, 274, 286; 5120^2 x 300 322, 329, 333);
+//     269, 274, 286; 5120^2 x 300 322, 329, 333).  Below K = 128 the memory is the
+//     bound and more workgroups keep it busier with C (8192^2 x 16 108, 140, 165;
+//     x 64 215, 223, 237; without C 68, 65, 68 and 198, 196, 192);
 //   * the others in 128x128 tiles from 5900^2 up, where three per CU at once fill
 //     (6144^3: 5558, 5407, 5479; 8192: 12893, 12620, 12588; not full: 7168: 8788,
 //     8782, 9090), and in 128x64 tiles at eight and more full rounds up to 4096^2
@@ -408,6 +410,7 @@ int valu_pick_cfg(int op, int R, int Cn, int K) {
     const int64_t rounds = (tiles(bm, bn) + cus - 1) / cus;
     return area / ((double)bm * bn * cus * rounds);
   };
+  if (op == 8 && K < 128) return CFG_S64;
   if (op == 8 && tiles(128, 128) > 3 * cus && fill(128, 128) >= 0.91) return CFG_L128;
   if (a <= 4096.0 * 4096.0 * 1.01)
     return tiles(128, 64) >= 8 * cus && fill(128, 64) >= 0.975 ? CFG_M128x64 : CFG_S64;

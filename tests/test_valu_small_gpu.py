@@ -98,6 +98,7 @@ def test_loop_uses_the_change_test(n):
 @pytest.mark.parametrize("op,m,n,k,cfg", [
     ("minus_square", 8192, 4096, 300, 0), ("minus_square", 5376, 5376, 300, 0),
     ("minus_square", 4608, 4608, 300, 1), ("minus_square", 5120, 5120, 128, 1),
+    ("minus_square", 8192, 8192, 64, 1), ("minus_square", 16384, 16384, 128, 0),
     ("min_plus", 3900, 3900, 512, 1), ("min_plus", 4096, 4096, 4096, 2),
     ("max_min", 2048, 8192, 1000, 2), ("max_min", 4100, 4100, 300, 1)])
 def test_tile_shape_by_full_rounds(op, m, n, k, cfg):
