@@ -7,9 +7,9 @@
 // v_mfma_f32_32x32x64_f8f6f4 sums the products in FP32, every term at least
 // 0.25 and none negative, so the sum is zero exactly when no term is 1.
 // Bounds: 65536 FP4 operations an instruction, 9.3 PFLOP/s measured with
-// operands in registers.  4096^3 at density 0.5 takes 42 us and 8192^3 287 us
-// (3.8 P ops/s, 43% of the matrix cores' cycles); the VALU form before it,
-// 32 (and, or) terms per v_and_or_b32, took 128 and 830 us.  What is left is
+// operands in registers.  4096^3 at density 0.5 takes 39 us and 8192^3 269 us
+// (4.1 P ops/s, 44% of the matrix cores' cycles); the VALU form before it,
+// 32 (and, or) terms per v_and_or_b32, took 124 and 830 us.  What is left is
 // the conversion of bits to FP4 (80 VALU and 82 scalar instructions per wave
 // and 128 k), which two waves per SIMD overlap only in part with 512 cycles
 // of products.

@@ -64,8 +64,8 @@ __attribute__((amdgpu_waves_per_eu(WAVES))) void srgemm_valu_kernel(
 // the epilogue.  Only where (+) is min or max, which is exact: regrouping the
 // terms changes no bit.  Bound: VALU issue at two waves per SIMD; four groups
 // of 256 threads with 4x4 outputs per lane (the split kernel below) read LDS
-// twice as often per term and meet at 1024-thread barriers: 1024^3 41 us, here
-// 36.  With more tiles a second wave per SIMD hides less than those groups do,
+// twice as often per term and meet at 1024-thread barriers: 1024^3 42 us, here
+// 38.  With more tiles a second wave per SIMD hides less than those groups do,
 // and so do the masked loads off the grid (1000x1000x700 33 us, 36 this way).
 constexpr int WT = 64, WTM = 8, WBK = 16;
 constexpr int WG = 8;  // waves per tile
